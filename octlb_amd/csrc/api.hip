@@ -191,7 +191,10 @@ struct octlb_dev {
   std::vector<SimConst> scm;      // constants per member
   SimConst* d_scm = nullptr;
   int* d_stat_tiles = nullptr;    // [nmembers + 1] stats-level tile offsets per member
-  int* d_stat_cells = nullptr;    // [nmembers + 1] statistic slots per member
+  int4* d_stat_chunk = nullptr;   // chunks of the reference-order sum (StatChunks)
+  int* d_stat_chunk_begin = nullptr;  // [nmembers + 1]
+  StatPart* d_stat_part = nullptr;
+  int stat_chunks = 0;
   int* d_step = nullptr;   // [2]: double-buffered coarse-step counter
   int step_slot = 0;       // slot holding the current step's time
   int* inc_next = nullptr; // next-step slot, handed to the step's first kernel
@@ -1081,8 +1084,14 @@ void octlb_dev::Prepare() {
     }
     d_stat_tiles = PAlloc<int>(nmembers + 1);
     Upload(d_stat_tiles, tiles_of, stream);
-    d_stat_cells = PAlloc<int>(nmembers + 1);
-    Upload(d_stat_cells, cells, stream);
+    std::vector<int> chunk_begin;
+    const std::vector<int4> chunk = StatChunks(cells, &chunk_begin);
+    stat_chunks = static_cast<int>(chunk.size());
+    d_stat_chunk = PAlloc<int4>(chunk.size());
+    Upload(d_stat_chunk, chunk, stream);
+    d_stat_chunk_begin = PAlloc<int>(chunk_begin.size());
+    Upload(d_stat_chunk_begin, chunk_begin, stream);
+    d_stat_part = PAlloc<StatPart>(chunk.size());
   }
   Upload(d_bt, bt, stream);
   Sync();
@@ -1347,7 +1356,9 @@ void octlb_dev::Level(int l) {
     }
     par[l] ^= 1;
     if (a.want_stats == 1) LaunchStatsFinalize<T>(d_stats, d_stat_tiles, nmembers, d_avg, stream);
-    if (a.want_stats == 2) LaunchStatsSequential(d_stat_val, d_stat_use, d_stat_cells, nmembers, d_avg, stream);
+    if (a.want_stats == 2)
+      LaunchStatsSequential(d_stat_val, d_stat_use, d_stat_chunk, d_stat_chunk_begin, stat_chunks, nmembers,
+                            d_stat_part, d_avg, stream);
   }
   if (fd_phase[3] > 0) {
     if (padded) {

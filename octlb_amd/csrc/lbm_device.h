@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "d3q19.h"
 #include "octlb_gpu.h"
 
@@ -468,12 +470,23 @@ __device__ __forceinline__ void CollideCell(T* f, int k, const SimConst& sc, con
 template <typename T>
 void LaunchTile(const TileArgs<T>& a, hipStream_t s);
 // ConstRho averages of the members: member m owns tiles [tile_begin[m],
-// tile_begin[m+1]) of the partial sums, or statistic slots [cell_begin[m],
-// cell_begin[m+1]) in the reference's order.
+// tile_begin[m+1]) of the partial sums.
 template <typename T>
 void LaunchStatsFinalize(const double* partial, const int* tile_begin, int members, double* avg, hipStream_t s);
-void LaunchStatsSequential(const double* val, const uint8_t* use, const int* cell_begin, int members, double* avg,
-                           hipStream_t s);
+// The reference-order sum goes by chunks of consecutive cells: (first cell,
+// end, member, cells of the member before it), member m owning chunks
+// [chunk_begin[m], chunk_begin[m + 1]); part holds one entry per chunk.
+struct StatPair {
+  long long d0, d1;  // what the chunk adds to an even / odd integer sum
+};
+struct StatPart {
+  StatPair p;
+  int count;
+  int e;  // exponent of the running sum the pair holds for
+};
+std::vector<int4> StatChunks(const std::vector<int>& cell_begin, std::vector<int>* chunk_begin);
+void LaunchStatsSequential(const double* val, const uint8_t* use, const int4* chunk, const int* chunk_begin,
+                           int nchunk, int members, StatPart* part, double* avg, hipStream_t s);
 void LaunchStepInc(const int* step, int* step_next, hipStream_t s);
 template <typename T>
 void LaunchInitEq(T* pops, const uint8_t* kind, int nb, const SimConst& sc, double rho0,
