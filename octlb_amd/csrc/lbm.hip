@@ -812,9 +812,6 @@ struct FdView {
   const T* cur;
   const T* post;
   const int* smap;      // this block's FD cell -> entry (or -1)
-  const T* lpre;        // LDS copy of the block ([19][512]) or nullptr
-  const T* lpost;       // LDS new values per FD slot ([slot][19])
-  const short* lsmap;   // LDS FD cell -> slot (or -1)
   const uint8_t* kind;
   const SimConst* sc;
   const double* org;
@@ -838,17 +835,6 @@ struct FdView {
   __device__ int Kind(int x, int y, int z) const { return kind[(x * sc->n + y) * sc->n + z]; }
   __device__ void Pops(int x, int y, int z, T* f) const {
     const int c = (x * sc->n + y) * sc->n + z;
-    if (lpre) {
-      const int e = lsmap[c];
-      if (e >= 0 && c < self) {
-#pragma unroll
-        for (int i = 0; i < kQ; ++i) f[i] = lpost[e * kQ + i];
-      } else {
-#pragma unroll
-        for (int i = 0; i < kQ; ++i) f[i] = lpre[i * kTileCells + c];
-      }
-      return;
-    }
     const int e = smap[c];
     if (e >= 0 && c < self) {
 #pragma unroll
@@ -947,50 +933,7 @@ struct FdView {
     ProxyRhoU(f, rho, u);
     return rho;
   }
-  __device__ void ComputeRhoU(int x, int y, int z, T& rho, T* u) const {
-    const int k = Kind(x, y, z);
-    if (k == kVelocity) {
-      Prescribed(x, y, z, u);
-      rho = ComputeRho(x, y, z);
-      return;
-    }
-    if (k == kPressure) {
-      rho = PrescribedRho(x, y, z);
-      int dir, ori;
-      if (!FlatInfo(sc->n, x, y, z, dir, ori)) {
-        u[0] = u[1] = u[2] = T(0);
-        return;
-      }
-      ComputeU(x - (dir == 0 ? ori : 0), y - (dir == 1 ? ori : 0), z - (dir == 2 ? ori : 0), u);
-      return;
-    }
-    T f[kQ];
-    Pops(x, y, z, f);
-    ProxyRhoU(f, rho, u);
-  }
-  __device__ void NormalGrad(int x, int y, int z, int axis, int normal, T* g) const {
-    const int ox = axis == 0 ? -normal : 0, oy = axis == 1 ? -normal : 0, oz = axis == 2 ? -normal : 0;
-    T u0[3], u1[3], u2[3];
-    ComputeU(x, y, z, u0);
-    ComputeU(x + ox, y + oy, z + oz, u1);
-    ComputeU(x + 2 * ox, y + 2 * oy, z + 2 * oz, u2);
-    for (int d = 0; d < 3; ++d)
-      g[d] = T(-normal) * ((-T(3) * u0[d] + T(4) * u1[d] - T(1) * u2[d]) / T(2));
-  }
-  __device__ void TangGrad(int x, int y, int z, int tx, int ty, int tz, T* g) const {
-    T up[3], um[3];
-    ComputeU(x + tx, y + ty, z + tz, up);
-    ComputeU(x - tx, y - ty, z - tz, um);
-    for (int d = 0; d < 3; ++d) g[d] = (up[d] - um[d]) / T(2);
-  }
 };
-
-template <typename T>
-__device__ inline void WriteFromPi(T* f, T rho, const T* u, const T* pi) {
-  const T usqr = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-#pragma unroll
-  for (int i = 0; i < kQ; ++i) f[i] = Feq(i, rho, u, usqr) + PiToFneq(i, pi);
-}
 
 // rho is r (rho for FP64, rho - 1 for FP32)
 template <typename T>
@@ -1004,138 +947,108 @@ __device__ inline void PiFromGrad(T rho, T omega, const T* dx, const T* dy, cons
   pi[4] = (dy[2] + dz[1]) * s;
 }
 
-// One FD boundary cell (ApplyInterpolatedVelocityBoundaryCells body).
-template <typename T, typename V>
-__device__ inline void FdCell(const V& v, int ix, int iy, int iz, T* fnew) {
-  const SimConst& sc = *v.sc;
-  const int n = sc.n;
-  const T omega = static_cast<T>(sc.omega);
-  const int xm = ix == 0, xp = ix == n - 1, ym = iy == 0, yp = iy == n - 1, zm = iz == 0, zp = iz == n - 1;
-  const int fc = xm + xp + ym + yp + zm + zp;
-  const int xn = xm ? -1 : (xp ? 1 : 0), yn = ym ? -1 : (yp ? 1 : 0), zn = zm ? -1 : (zp ? 1 : 0);
-  T pi[6];
-  if (fc == 3) {
-    // ApplyCornerBoundary (:638-685)
-    const T r100 = v.ComputeRho(ix - xn, iy, iz);
-    const T r010 = v.ComputeRho(ix, iy - yn, iz);
-    const T r001 = v.ComputeRho(ix, iy, iz - zn);
-    const T r200 = v.ComputeRho(ix - 2 * xn, iy, iz);
-    const T r020 = v.ComputeRho(ix, iy - 2 * yn, iz);
-    const T r002 = v.ComputeRho(ix, iy, iz - 2 * zn);
-    const T rho = T(4) / T(9) * (r001 + r010 + r100) - T(1) / T(9) * (r002 + r020 + r200);
-    T dx[3], dy[3], dz[3], u[3];
-    v.NormalGrad(ix, iy, iz, 0, xn, dx);
-    v.NormalGrad(ix, iy, iz, 1, yn, dy);
-    v.NormalGrad(ix, iy, iz, 2, zn, dz);
-    v.ComputeU(ix, iy, iz, u);
-    PiFromGrad(rho, omega, dx, dy, dz, pi);
-    WriteFromPi(fnew, rho, u, pi);
-  } else if (fc == 2) {
-    // ApplyEdgeBoundary (:687-752)
-    int plane, n1, n2;
-    if (xn != 0 && yn != 0) {
-      plane = 2;
-      n1 = xn;
-      n2 = yn;
-    } else if (xn != 0 && zn != 0) {
-      plane = 1;
-      n1 = xn;
-      n2 = zn;
-    } else {
-      plane = 0;
-      n1 = yn;
-      n2 = zn;
-    }
-    const int d1 = (plane + 1) % 3, d2 = (plane + 2) % 3;
-    T rs[4];
-    const int st[4][2] = {{1, 0}, {0, 1}, {2, 0}, {0, 2}};
-    for (int q = 0; q < 4; ++q) {
-      int o[3] = {0, 0, 0};
-      o[d1] = -n1 * st[q][0];
-      o[d2] = -n2 * st[q][1];
-      rs[q] = v.ComputeRho(ix + o[0], iy + o[1], iz + o[2]);
-    }
-    const T rho = T(2) / T(3) * (rs[1] + rs[0]) - T(1) / T(6) * (rs[3] + rs[2]);
-    T g[3][3];
-    for (int p = 0; p < 3; ++p)
-      for (int q = 0; q < 3; ++q) g[p][q] = T(0);
-    v.TangGrad(ix, iy, iz, plane == 0, plane == 1, plane == 2, g[plane]);
-    v.NormalGrad(ix, iy, iz, d1, n1, g[d1]);
-    v.NormalGrad(ix, iy, iz, d2, n2, g[d2]);
-    T u[3];
-    v.ComputeU(ix, iy, iz, u);
-    const T s = -RhoOf(rho) / T(3) / omega;
-    pi[0] = T(2) * g[0][0] * s;
-    pi[3] = T(2) * g[1][1] * s;
-    pi[5] = T(2) * g[2][2] * s;
-    pi[1] = (g[0][1] + g[1][0]) * s;
-    pi[2] = (g[0][2] + g[2][0]) * s;
-    pi[4] = (g[1][2] + g[2][1]) * s;
-    WriteFromPi(fnew, rho, u, pi);
-  } else {
-    // ApplyPlaneFdBoundary (:570-636)
-    int face = OCTLB_XMIN;
-    if (xp) {
-      face = OCTLB_XMAX;
-    } else if (yp) {
-      face = OCTLB_YMAX;
-    } else if (ym) {
-      face = OCTLB_YMIN;
-    } else if (zp) {
-      face = OCTLB_ZMAX;
-    } else if (zm) {
-      face = OCTLB_ZMIN;
-    }
-    const int direction = face / 2, orientation = (face & 1) ? 1 : -1;
-    T rho, u[3];
-    v.ComputeRhoU(ix, iy, iz, rho, u);
-    T dx[3] = {T(0), T(0), T(0)}, dy[3] = {T(0), T(0), T(0)}, dz[3] = {T(0), T(0), T(0)};
-    if (direction == 0) {
-      v.NormalGrad(ix, iy, iz, 0, orientation, dx);
-      v.TangGrad(ix, iy, iz, 0, 1, 0, dy);
-      v.TangGrad(ix, iy, iz, 0, 0, 1, dz);
-    } else if (direction == 1) {
-      v.TangGrad(ix, iy, iz, 1, 0, 0, dx);
-      v.NormalGrad(ix, iy, iz, 1, orientation, dy);
-      v.TangGrad(ix, iy, iz, 0, 0, 1, dz);
-    } else {
-      v.TangGrad(ix, iy, iz, 1, 0, 0, dx);
-      v.TangGrad(ix, iy, iz, 0, 1, 0, dy);
-      v.NormalGrad(ix, iy, iz, 2, orientation, dz);
-    }
-    PiFromGrad(rho, omega, dx, dy, dz, pi);
-    WriteFromPi(fnew, rho, u, pi);
-  }
-}
+// Velocity set and weights by run-time index.
+__constant__ int kCxT[kQ] = {0, -1, 0, 0, -1, -1, -1, -1, 0, 0, 1, 0, 0, 1, 1, 1, 1, 0, 0};
+__constant__ int kCyT[kQ] = {0, 0, -1, 0, -1, 1, 0, 0, -1, -1, 0, 1, 0, 1, -1, 0, 0, 1, 1};
+__constant__ int kCzT[kQ] = {0, 0, 0, -1, 0, 0, -1, 1, -1, 1, 0, 0, 1, 0, 0, 1, -1, 1, -1};
+__constant__ int kWDenT[kQ] = {3, 18, 18, 18, 36, 36, 36, 36, 36, 36, 18, 18, 18, 36, 36, 36, 36, 36, 36};
 
 template <typename T>
-__global__ void KFd(FdArgs<T> a, int begin, int count) {
+__device__ inline T FdPopulation(const int* c, T t, T rho, const T* u, T usqr, const T* pi);
+
+// FD boundary cells of padded blocks (ApplyInterpolatedVelocityBoundaryCells
+// body, interpolated_velocity.h:950-1036), 16 lanes per cell.  A cell reads
+// the velocity at itself and at two cells per axis and the density at up to
+// six cells, each from 19 populations or a walk to other cells: a chain of
+// latencies, with few cells per phase.  So every lane evaluates one of these
+// points (0..5 the axes' two points, 6 the cell itself, 8..13 the densities)
+// and the gradients come together by shuffles; one thread per cell, point
+// after point, took 43.5 us a phase on a 64^3 block, this takes 12.2 us.
+constexpr int kFdLanes = 16;
+constexpr int kFdThreads = 256;
+template <typename T>
+__global__ __launch_bounds__(kFdThreads) void KFd(FdArgs<T> a, int begin, int count) {
   BumpStep(a.step, a.step_next);
-  const int e = begin + static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-  if (e >= begin + count) return;
+  const int g = static_cast<int>(blockIdx.x * kFdThreads + threadIdx.x) / kFdLanes;
+  const int lane = threadIdx.x % kFdLanes;
+  const bool live = g < count;  // the last groups repeat a cell: every lane takes part in the shuffles
+  const int e = begin + (live ? g : count - 1);
   const int b = a.cells[e].x, c = a.cells[e].y;
   const SimConst& sc = a.sc;
   const int n = sc.n;
-  const int ix = c / (n * n), iy = (c / n) % n, iz = c % n;
-  const int lvl = a.level[b];
-  const T* cur = (a.par.v[lvl] ? a.pops1 : a.pops0) + static_cast<size_t>(b) * kQ * sc.plane;
+  const int pos[3] = {c / (n * n), (c / n) % n, c % n};
   FdView<T> v;
-  v.cur = cur;
+  v.cur = (a.par.v[a.level[b]] ? a.pops1 : a.pops0) + static_cast<size_t>(b) * kQ * sc.plane;
   v.post = a.post;
   v.smap = a.smap + static_cast<size_t>(a.fd_index[b]) * sc.ncore;
-  v.lpre = nullptr;
-  v.lpost = nullptr;
-  v.lsmap = nullptr;
   v.kind = a.kind + static_cast<size_t>(b) * sc.ncore;
   v.sc = &a.sc;
   v.org = a.bt[b].origin;
   v.cw = a.bt[b].cw;
   v.t = static_cast<double>(*a.step);
   v.self = c;
-  T fnew[kQ];
-  FdCell<T>(v, ix, iy, iz, fnew);
-  T* po = a.post + static_cast<size_t>(e) * kQ;
-  for (int i = 0; i < kQ; ++i) po[i] = fnew[i];
+
+  // normal[a]: the outward normal whose one-sided difference (ApplyPlaneFd-,
+  // ApplyEdge-, ApplyCornerBoundary, :570-752) gives the gradient along axis
+  // a; 0 for the central difference along a tangential axis
+  int on[3];
+  for (int d = 0; d < 3; ++d) on[d] = pos[d] == 0 ? -1 : (pos[d] == n - 1 ? 1 : 0);
+  const int fc = (on[0] != 0) + (on[1] != 0) + (on[2] != 0);
+  int normal[3] = {on[0], on[1], on[2]};
+  if (fc == 0) normal[0] = -1;  // a cell on no face counts as the x- face's (:1013)
+  if (fc == 2 && on[1] == 0) {  // x-z edges: axis z takes the x side's sign and x the z side's (:700-713)
+    normal[0] = on[2];
+    normal[2] = on[0];
+  }
+  T r = RestR<T>(), u[3] = {T(0), T(0), T(0)};
+  if (lane < 7) {
+    int at[3] = {pos[0], pos[1], pos[2]};
+    if (lane < 6) {
+      const int ax = lane >> 1, far = lane & 1;
+      const int nrm = ax == 0 ? normal[0] : (ax == 1 ? normal[1] : normal[2]);
+      const int step = nrm != 0 ? -nrm * (1 + far) : (far ? -1 : 1);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) at[d] += d == ax ? step : 0;
+    }
+    v.ComputeU(at[0], at[1], at[2], u);
+  } else if (lane >= 8 && lane < 8 + (fc == 3 ? 6 : (fc == 2 ? 4 : 1))) {
+    int at[3] = {pos[0], pos[1], pos[2]};
+    if (fc >= 2) {
+      // corner: lanes r100, r010, r001, r200, r020, r002; edge: the two
+      // normal axes d1 = plane + 1, d2 = plane + 2 (mod 3) at one and two steps
+      const int q = lane - 8;
+      const int plane = on[0] == 0 ? 0 : (on[1] == 0 ? 1 : 2);
+      const int ax = fc == 3 ? q % 3 : (plane + 1 + (q & 1)) % 3;
+      const int far = fc == 3 ? q / 3 : q >> 1;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) at[d] -= d == ax ? normal[d] * (1 + far) : 0;
+    }
+    r = v.ComputeRho(at[0], at[1], at[2]);
+  }
+
+  T us[3], G[3][3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) us[d] = __shfl(u[d], 6, kFdLanes);
+#pragma unroll
+  for (int ax = 0; ax < 3; ++ax)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const T u1 = __shfl(u[d], 2 * ax, kFdLanes), u2 = __shfl(u[d], 2 * ax + 1, kFdLanes);
+      G[ax][d] = normal[ax] != 0 ? T(-normal[ax]) * ((-T(3) * us[d] + T(4) * u1 - T(1) * u2) / T(2)) : (u1 - u2) / T(2);
+    }
+  T rs[6];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) rs[q] = __shfl(r, 8 + q, kFdLanes);
+  const T rho = fc == 3 ? T(4) / T(9) * (rs[2] + rs[1] + rs[0]) - T(1) / T(9) * (rs[5] + rs[4] + rs[3])
+                        : (fc == 2 ? T(2) / T(3) * (rs[1] + rs[0]) - T(1) / T(6) * (rs[3] + rs[2]) : rs[0]);
+  T pi[6];
+  PiFromGrad(rho, static_cast<T>(sc.omega), G[0], G[1], G[2], pi);
+  const T usqr = us[0] * us[0] + us[1] * us[1] + us[2] * us[2];
+  if (!live) return;
+  for (int i = lane; i < kQ; i += kFdLanes) {
+    const int ci[3] = {kCxT[i], kCyT[i], kCzT[i]};
+    a.post[static_cast<size_t>(e) * kQ + i] = FdPopulation<T>(ci, T(1) / T(kWDenT[i]), rho, us, usqr, pi);
+  }
 }
 
 // Blocked mode: one workgroup per boundary block.  Every cell's density and
@@ -1221,11 +1134,6 @@ __device__ inline T FdRhoOf(int k, const T* f, const T* pu, const SimConst& sc, 
 
 // Runtime-index forms of Feq / PiToFneq for the (cell, population) task
 // loops; same operations in the same order as the compile-time versions.
-__constant__ int kCxT[kQ] = {0, -1, 0, 0, -1, -1, -1, -1, 0, 0, 1, 0, 0, 1, 1, 1, 1, 0, 0};
-__constant__ int kCyT[kQ] = {0, 0, -1, 0, -1, 1, 0, 0, -1, -1, 0, 1, 0, 1, -1, 0, 0, 1, 1};
-__constant__ int kCzT[kQ] = {0, 0, 0, -1, 0, 0, -1, 1, -1, 1, 0, 0, 1, 0, 0, 1, -1, 1, -1};
-__constant__ int kWDenT[kQ] = {3, 18, 18, 18, 36, 36, 36, 36, 36, 36, 18, 18, 18, 36, 36, 36, 36, 36, 36};
-
 template <typename T>
 __device__ inline T FdPopulation(const int* c, T t, T rho, const T* u, T usqr, const T* pi) {
   T cu = T(0);
@@ -2021,7 +1929,8 @@ template <typename T>
 void LaunchFd(const FdArgs<T>& a, const int* phase_begin, hipStream_t s) {
   for (int ph = 0; ph < 3; ++ph) {
     const int cnt = phase_begin[ph + 1] - phase_begin[ph];
-    if (cnt > 0) hipLaunchKernelGGL(KFd<T>, Grid(cnt, 128), dim3(128), 0, s, a, phase_begin[ph], cnt);
+    if (cnt > 0) hipLaunchKernelGGL(KFd<T>, Grid(static_cast<long long>(cnt) * kFdLanes, kFdThreads), dim3(kFdThreads), 0, s, a,
+                         phase_begin[ph], cnt);
   }
   const int total = phase_begin[3];
   if (total > 0) hipLaunchKernelGGL(KFdCommit<T>, Grid(total, 256), dim3(256), 0, s, a, total);
