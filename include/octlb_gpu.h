@@ -345,7 +345,7 @@ int octlb_build_links(int32_t num_blocks, int32_t n, const double* bounds, const
  * but every array (bounds, material, triangles in; links, q out) is a
  * device pointer the caller owns, the work is queued on `stream` (null: the
  * default stream) and the call allocates nothing: its scratch is a static
- * device array of about 10.9 MB per GPU, held until the process ends.
+ * device array of about 11.7 MB per GPU, held until the process ends.
  * Limits: num_blocks <= 16384 and at most 65536 candidate cells (fluid cells
  * with a solid-like in-block neighbour); beyond either, OCTLB_EINVAL (the
  * block limit before any device work, the candidate limit after the
