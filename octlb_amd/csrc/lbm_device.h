@@ -36,6 +36,15 @@ namespace octlb {
 #define OCTLB_CONST_TABLE
 #endif
 
+// Gives a branch its own copies of rho and u, as far as the compiler can tell.
+// Without them it forms the terms that the three collisions share ahead of the
+// branches and holds them all: 19 registers more than FP32 has.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define OCTLB_OWN_TERMS(name, r, u) asm volatile(name : "+v"(r), "+v"((u)[0]), "+v"((u)[1]), "+v"((u)[2]))
+#else
+#define OCTLB_OWN_TERMS(name, r, u)
+#endif
+
 constexpr int kTile = 8;                       // tile edge (cells)
 constexpr int kBox = kTile + 2;                // tile + one-cell apron
 constexpr int kBoxCells = kBox * kBox * kBox;  // 1000
@@ -412,9 +421,9 @@ __device__ __forceinline__ void CollideCell(T* f, int k, const SimConst& sc, con
   const double cw = og.cw;
   const T omega = static_cast<T>(sc.omega);
   if (k == kBulk) {
+    T rho, u[3];
+    ProxyRhoU(f, rho, u);
     if (sc.const_rho) {
-      T rho, u[3];
-      ProxyRhoU(f, rho, u);
       if (want) {
         if constexpr (kShiftedArith<T>) {
           ssum += 1.0 + (static_cast<double>(rho) - static_cast<double>(avg));  // rho + (1 - avg)
@@ -423,13 +432,13 @@ __device__ __forceinline__ void CollideCell(T* f, int k, const SimConst& sc, con
         }
         scnt += 1;
       }
+      OCTLB_OWN_TERMS("; const rho", rho, u);
       ConstRhoBgk(f, omega, avg, rho, u);
     } else if (sc.handler == OCTLB_HANDLER_CONCRETE) {
-      T rho, u[3];
-      ProxyRhoU(f, rho, u);
+      OCTLB_OWN_TERMS("; concrete", rho, u);
       OlbBgk(f, rho, u, omega);
     } else {
-      CollideBgkAt(f, omega);
+      CollideBgkAt(f, rho, u, omega);
     }
     return;
   }
