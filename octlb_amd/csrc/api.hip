@@ -10,7 +10,6 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
-#include <unordered_map>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -137,6 +136,8 @@ struct octlb_dev {
   // octlb_dev_autotune.
   int variant = 1;
   int npush_blocks = 0;
+  int* d_push_blocks = nullptr;  // push-class blocks, level by level
+  int push_tiles[kMaxLevels] = {};
   // ---- device
   hipStream_t stream = nullptr;
   void* pops[2] = {nullptr, nullptr};
@@ -608,7 +609,7 @@ void octlb_dev::Build(const octlb_topology* t, const octlb_params* p) {
   }
   d_level = Alloc<int>(nb);
   Upload(d_level, level, stream);
-  d_stats = Alloc<double>(2 * tiles.size());
+  d_stats = Alloc<double>(2 * tiles.size() * (padded ? 1 : kTile));
   fast_stats = p->fast_stats != 0;
   if (sc.const_rho && !fast_stats) {
     d_stat_val = Alloc<double>(static_cast<size_t>(nb) * ncore);
@@ -703,9 +704,9 @@ void octlb_dev::Prepare() {
       bool plain = true;
       for (int c = 0; c < ncore; ++c) {
         const size_t cg = static_cast<size_t>(b) * ncore + c;
-        bool need = kb[c] == kSolid || ReflectsOnPull(kb[c]) || qmask[cg] != 0;
+        bool need = sc.bouzidi && (kb[c] == kSolid || ReflectsOnPull(kb[c]) || qmask[cg] != 0);
         const int ix = c / (n * n), iy = (c / n) % n, iz = c % n;
-        for (int i = 1; i < kQ && !need; ++i) {
+        for (int i = 1; i < kQ && !need && sc.bouzidi; ++i) {
           const int x = ix - Cx(i), y = iy - Cy(i), z = iz - Cz(i);
           if (x < 0 || x >= n || y < 0 || y >= n || z < 0 || z >= n) continue;
           const int sk = kb[(x * n + y) * n + z];
@@ -822,17 +823,19 @@ void octlb_dev::Prepare() {
   // every cell streams by the plain pull, its 18 halo parts are all exchanged
   // at its level (no shell, no coupling, no FD face), nothing reads its
   // post-collide values between collide and stream (no drag snapshot) and no
-  // coupling point writes it.  Reference-order ConstRho statistics keep one
-  // block per tile, so they keep the pull scheme.
+  // coupling point writes it.  Blocks with a shell push as well as any other
+  // cell by cell, but their shell's own streaming needs the re-collided cells
+  // of the exchanged parts next to it, five more waves beside the block's
+  // eight: 23,456 wall blocks of an ensemble took 926 us that way and 756 us
+  // as pull tiles (FP32).
   npush_blocks = 0;
   if (!padded) {
-    const bool push_ok = variant == 1 && !(sc.const_rho && !fast_stats);
     std::vector<char> is_push(nb, 0);
     for (int b = 0; b < nb; ++b) {
       BlockTab& r = bt[b];
       for (int k = 0; k < 18; ++k) r.push_to[k] = -1;
-      if (!push_ok) continue;
-      bool ok = (r.flags & kFlagPlain) && !(r.flags & (kFlagShellLive | kFlagDrag | kFlagProlong | kFlagLinks));
+      bool ok = variant == 1 && (r.flags & kFlagPlain) &&
+                !(r.flags & (kFlagShellLive | kFlagDrag | kFlagProlong | kFlagLinks));
       for (int k = 0; k < 18 && ok; ++k) ok = r.nbr[k] >= 0;
       is_push[b] = ok ? 1 : 0;
     }
@@ -858,31 +861,42 @@ void octlb_dev::Prepare() {
       for (int k = 0; k < 18; ++k)
         if (bt[b].push_to[k] >= 0) bt[b].flags |= kFlagPushOut;
     }
-    // tiles: per level in visiting order; consecutive push-class blocks of
-    // one ensemble member pair up in a push tile
+    // tiles, per level in visiting order: the wave tasks of consecutive
+    // push-class blocks fill a push tile.  Pull tiles read what their push
+    // neighbours read, and find it in L2 only if both run at about the same
+    // time: with the push tasks in a launch of their own, which needs no LDS,
+    // the 64-member ensemble took 1355 us a step where this order takes 1270
+    // (FP32), the 2-level cylinder's finest level 52.8 against 47.8 (FP64).
+    std::vector<int> push_blocks;
     tiles.clear();
     for (int l = 0; l <= max_level; ++l) {
       tile_begin[l] = static_cast<int>(tiles.size());
-      int pending = -1;
+      push_tiles[l] = 0;
+      int begun = static_cast<int>(push_blocks.size()) * kTile;  // first task without a tile
+      auto tile = [&](int at_least) {
+        for (int left; (left = static_cast<int>(push_blocks.size()) * kTile - begun) >= at_least; ++push_tiles[l]) {
+          tiles.push_back(Tile{begun, std::min(kTaskWaves, left), 1, 0});
+          begun += std::min(kTaskWaves, left);
+        }
+      };
       for (int bi = 0; bi < nb; ++bi) {
         const int b = block_order[bi];
         if (level[b] != l) continue;
-        if (!is_push[b]) {
+        if (is_push[b]) {
+          push_blocks.push_back(b);
+          tile(kTaskWaves);
+        } else {
           tiles.push_back(Tile{b, 0, 0, 0});
-          continue;
         }
-        if (pending >= 0 && bt[pending].member == bt[b].member) {
-          tiles.push_back(Tile{pending, b, 1, 0});
-          pending = -1;
-          continue;
-        }
-        if (pending >= 0) tiles.push_back(Tile{pending, -1, 1, 0});
-        pending = b;
       }
-      if (pending >= 0) tiles.push_back(Tile{pending, -1, 1, 0});
+      tile(1);
       tile_count[l] = static_cast<int>(tiles.size()) - tile_begin[l];
     }
+    d_tiles = PAlloc<Tile>(tiles.size());
     Upload(d_tiles, tiles, stream);
+    d_push_blocks = PAlloc<int>(push_blocks.size());
+    Upload(d_push_blocks, push_blocks, stream);
+    Sync();  // the tables above leave scope
   }
   // ---- post-stream FD cell lists (concrete handler, tree-boundary blocks)
   std::vector<int2> fd_cells[3];
@@ -1056,8 +1070,8 @@ void octlb_dev::Prepare() {
   {
     const int l = max_level;
     const int tpb = padded ? ((NP + kTile - 1) / kTile) * ((NP + kTile - 1) / kTile) * ((NP + kTile - 1) / kTile) : 1;
-    // partial-sum slots of the member's blocks (blocked mode: one per block,
-    // in visiting order; padded mode: one per tile)
+    // partial-sum slots of the member's blocks (blocked mode: one per x plane
+    // of each block, in visiting order; padded mode: one per tile)
     std::vector<int> tiles_of(nmembers + 1, 0);
     int prev = 0;
     if (padded) {
@@ -1082,6 +1096,8 @@ void octlb_dev::Prepare() {
       tiles_of[m + 1] += tiles_of[m];
       cells[m + 1] = tiles_of[m + 1] / tpb * ncore;
     }
+    if (!padded)
+      for (int& t : tiles_of) t *= kTile;  // a partial per x plane
     d_stat_tiles = PAlloc<int>(nmembers + 1);
     Upload(d_stat_tiles, tiles_of, stream);
     std::vector<int> chunk_begin;
@@ -1149,6 +1165,8 @@ TileArgs<T> octlb_dev::MakeTileArgs(int l) {
   TileArgs<T> a{};
   a.tiles = d_tiles + tile_begin[l];
   a.ntiles = tile_count[l];
+  a.npush = padded ? 0 : push_tiles[l];
+  a.push_blocks = d_push_blocks;
   a.bt = d_bt;
   a.kind = d_kind;
   a.rule = d_rule;

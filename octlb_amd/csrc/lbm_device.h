@@ -36,6 +36,10 @@ namespace octlb {
 #define OCTLB_CONST_TABLE
 #endif
 
+// A condition that most waves find false: what it guards should take the
+// spills, not the path beside it.
+#define OCTLB_RARE(cond) (__builtin_expect(static_cast<bool>(cond), 0))
+
 // Gives a branch its own copies of rho and u, as far as the compiler can tell.
 // Without them it forms the terms that the three collisions share ahead of the
 // branches and holds them all: 19 registers more than FP32 has.
@@ -145,14 +149,17 @@ struct BlockTab {
   double cw;
 };
 
-// blocked mode: block = the tile's block; ox = second block of a push tile
-// (-1: none), oy = 1 for a push tile (two push-class blocks, one per half
-// of the workgroup), 0 for a pull tile.  padded mode: ox, oy, oz = origin
-// of the tile in the padded box.
+// blocked mode: oy = 0 for a pull tile of `block`; oy = 1 for a push tile:
+// `block` = its first wave task, ox = how many (at most kTaskWaves).  padded
+// mode: ox, oy, oz = origin of the tile in the padded box.
 struct Tile {
   int block;
   int ox, oy, oz;
 };
+
+// Work of one wave of a push tile: task t = x plane t % kTile of the
+// push-class block push_blocks[t / kTile].
+constexpr int kTaskWaves = 16;
 
 struct ParArray {
   int v[kMaxLevels];
@@ -195,6 +202,8 @@ template <typename T>
 struct TileArgs {
   const Tile* tiles;
   int ntiles;
+  int npush;              // push tiles among them
+  const int* push_blocks; // push-class blocks, level by level in visiting order
   const BlockTab* bt;
   const uint8_t* kind;
   const uint8_t* rule;    // per core cell: 1 = some pull-stream rule beyond the plain pull applies
@@ -208,7 +217,7 @@ struct TileArgs {
   const uint32_t* dmask;
   const int* doff;
   T* snap;
-  double* stats;          // [blocks*2] partial sums per block of the level (want_stats == 1)
+  double* stats;          // want_stats == 1: partial (sum, count) per x plane of each block of the level (padded: per tile)
   const int* block_rank;  // block -> its index among its level's blocks in visiting order
   double* stat_val;       // per-cell statistic in reference order (want_stats == 2)
   uint8_t* stat_use;
@@ -420,7 +429,7 @@ __device__ __forceinline__ void CollideCell(T* f, int k, const SimConst& sc, con
   const double org[3] = {og.x, og.y, og.z};
   const double cw = og.cw;
   const T omega = static_cast<T>(sc.omega);
-  if (k == kBulk) {
+  if (!OCTLB_RARE(k != kBulk)) {
     T rho, u[3];
     ProxyRhoU(f, rho, u);
     if (sc.const_rho) {
