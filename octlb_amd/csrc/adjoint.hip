@@ -37,11 +37,17 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <functional>
+#include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -84,6 +90,36 @@ __device__ __forceinline__ int XcdWg(int w, int n) {
 constexpr int kN = 8, kNP = 10, kNS = kNP * kNP * kNP, kNC = kN * kN * kN;
 constexpr int kThreads = 128;
 constexpr uint8_t kHalo = 255;  // kind of a halo slot: carried, never collided
+
+// body(k) for k in [0, count), spread over the host's threads (at most 16);
+// what a body throws is thrown here.
+template <typename F>
+void ParallelFor(int count, F&& body) {
+  constexpr int kChunk = 16;
+  const int want = std::min({16, static_cast<int>(std::thread::hardware_concurrency()), count / kChunk});
+  std::atomic<int> next{0};
+  std::exception_ptr failed;
+  std::mutex failed_mu;
+  auto run = [&] {
+    try {
+      for (int k0; (k0 = next.fetch_add(kChunk)) < count;)
+        for (int k = k0; k < std::min(k0 + kChunk, count); ++k) body(k);
+    } catch (...) {
+      std::lock_guard<std::mutex> lock(failed_mu);
+      if (!failed) failed = std::current_exception();
+      next = count;
+    }
+  };
+  std::vector<std::thread> threads;
+  try {
+    while (static_cast<int>(threads.size()) + 1 < want) threads.emplace_back(run);
+  } catch (const std::system_error&) {
+    // fewer threads than wanted: those there are, and this one, do the work
+  }
+  run();
+  for (std::thread& th : threads) th.join();
+  if (failed) std::rethrow_exception(failed);
+}
 
 struct AdjLink {
   int row;      // output entry
@@ -794,25 +830,74 @@ struct octlb_adj {
     omega = t.omega;
     prec = t.prec;
     selem = prec == 32 ? sizeof(float) : sizeof(double);
-    const long long nfull = static_cast<long long>(nb) * kQ * kNS;
-    if (nfull >= (1ll << 31)) throw std::invalid_argument("adjoint: too many blocks");
+    if (static_cast<long long>(nb) * kQ * kNS >= (1ll << 31)) throw std::invalid_argument("adjoint: too many blocks");
     origin_cw = t.origin_cw;
-    auto kind = [&](int b, int ix, int iy, int iz) {
+    auto kind = [&](int b, int ix, int iy, int iz) -> int {
       return t.kinds[static_cast<size_t>(b) * kNC + (ix * kN + iy) * kN + iz];
     };
-    std::unordered_map<int64_t, double> qmap;
-    for (size_t k = 0; k < t.link_key.size(); ++k) qmap[t.link_key[k]] = t.link_q[k];
-    // ---- rows of M over the full halo view: stream_block
-    // (block_lattice.cpp:503-720) after the exchange
-    auto resolve = [&](int b, int slot, int pop) {
-      const int hs = t.halo_src[static_cast<size_t>(b) * kNS + slot];
-      const int sb = hs >= 0 ? hs / kNS : b, ss = hs >= 0 ? hs % kNS : slot;
-      return (sb * kQ + pop) * kNS + ss;
-    };
-    auto in_np = [](int v) { return v >= 0 && v < kNP; };
+    std::vector<std::pair<int64_t, double>> q(t.link_key.size());
+    for (size_t k = 0; k < q.size(); ++k) q[k] = {t.link_key[k], t.link_q[k]};
+    std::stable_sort(q.begin(), q.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
     auto in_core = [](int v) { return v >= 0 && v < kN; };
-    std::vector<int> srcf(static_cast<size_t>(nfull));
-    std::vector<AdjLink> links;
+    auto core_slot = [&](int slot) {
+      return in_core(slot / (kNP * kNP) - 1) && in_core(slot / kNP % kNP - 1) && in_core(slot % kNP - 1);
+    };
+    // ---- a row of M over the full halo view, stream_block
+    // (block_lattice.cpp:503-720) after the exchange: the source of population
+    // i at a slot, or (link) the two sources and the fraction of a Bouzidi pull
+    struct Row {
+      int b, slot, pop;  // source
+      bool link, upper;
+      int ob, oslot;     // link: the other source (population i of the row)
+      int64_t key;
+      double q;
+    };
+    auto resolve = [&](int b, int slot, int* sb, int* ss) {
+      const int hs = t.halo_src[static_cast<size_t>(b) * kNS + slot];
+      *sb = hs >= 0 ? hs / kNS : b;
+      *ss = hs >= 0 ? hs % kNS : slot;
+    };
+    auto row = [&](int b, bool plain, int slot, int i) {
+      Row r{b, slot, i, false, false, 0, 0, 0, 0.0};
+      const int off = (Cx(i) * kNP + Cy(i)) * kNP + Cz(i);
+      const int hx = slot / (kNP * kNP), hy = slot / kNP % kNP, hz = slot % kNP;
+      const bool core = in_core(hx - 1) && in_core(hy - 1) && in_core(hz - 1);
+      if (!core || plain) {
+        // a core cell's source is never beyond the halo; a halo slot's wraps
+        const int s = slot - off;
+        resolve(b, s < 0 ? s + kNS : (s >= kNS ? s - kNS : s), &r.b, &r.slot);
+        return r;
+      }
+      const int k = kind(b, hx - 1, hy - 1, hz - 1);
+      if (k == kSolid) return r;
+      const int sx = hx - Cx(i) - 1, sy = hy - Cy(i) - 1, sz = hz - Cz(i) - 1;
+      const bool s_core = in_core(sx) && in_core(sy) && in_core(sz);
+      if (ReflectsOnPull(k) && !s_core) {
+        r.pop = Opp(i);
+        return r;
+      }
+      const int sk = s_core ? kind(b, sx, sy, sz) : kBulk;
+      if (sk == kSolid || sk == kBouzidi) {
+        r.pop = Opp(i);
+        r.key = (static_cast<int64_t>(b) * kNC + ((hx - 1) * kN + hy - 1) * kN + hz - 1) * kQ + i;
+        // of a link given twice the later fraction counts
+        const auto it = std::upper_bound(q.begin(), q.end(), r.key, [](int64_t k, const auto& x) { return k < x.first; });
+        const double qf = it == q.begin() || (it - 1)->first != r.key ? 1.0 : (it - 1)->second;
+        if (qf > 1.0e-10 && qf < 1.0 - 1.0e-10) {
+          const int nx = hx + Cx(i) - 1, ny = hy + Cy(i) - 1, nz = hz + Cz(i) - 1;
+          const int nk = in_core(nx) && in_core(ny) && in_core(nz) ? kind(b, nx, ny, nz) : kBulk;
+          r.link = true;
+          r.upper = qf >= 0.5 - 1.0e-14;
+          r.q = qf;
+          r.ob = b;
+          r.oslot = slot;
+          if (r.upper && nk == kBulk) resolve(b, slot + off, &r.ob, &r.oslot);
+        }
+        return r;
+      }
+      resolve(b, slot - off, &r.b, &r.slot);
+      return r;
+    };
     // blocks in level order (a stable sort: one level keeps the block order),
     // so that every level's cells, entries and links are contiguous ranges
     border.resize(nb);
@@ -821,263 +906,240 @@ struct octlb_adj {
       std::stable_sort(border.begin(), border.end(), [&](int a, int c) { return t.level[a] < t.level[c]; });
     const int nlev = t.level.empty() ? 1 : 1 + *std::max_element(t.level.begin(), t.level.end());
     auto lvl = [&](int b) { return t.level.empty() ? 0 : t.level[b]; };
-    lv_link.assign(nlev + 1, 0);
-    for (int bi = 0; bi < nb; ++bi) {
-      const int b = border[bi];
-      lv_link[lvl(b) + 1] = -1;  // filled below
-      for (int hx = 0; hx < kNP; ++hx)
-        for (int hy = 0; hy < kNP; ++hy)
-          for (int hz = 0; hz < kNP; ++hz) {
-            const int ix = hx - 1, iy = hy - 1, iz = hz - 1;
-            const bool core = in_core(ix) && in_core(iy) && in_core(iz);
-            const int dst = (hx * kNP + hy) * kNP + hz;
-            for (int i = 0; i < kQ; ++i) {
-              const int e = (b * kQ + i) * kNS + dst;
-              const int sx = hx - Cx(i), sy = hy - Cy(i), sz = hz - Cz(i);
-              const bool s_in = in_np(sx) && in_np(sy) && in_np(sz);
-              if (!core) {
-                int s;
-                if (s_in) {
-                  s = (sx * kNP + sy) * kNP + sz;
-                } else {
-                  const int off = Cx(i) * kNP * kNP + Cy(i) * kNP + Cz(i);
-                  s = ((dst - off) % kNS + kNS) % kNS;
-                }
-                srcf[e] = resolve(b, s, i);
-                continue;
-              }
-              const int k = kind(b, ix, iy, iz);
-              if (k == kSolid) {
-                srcf[e] = e;
-                continue;
-              }
-              const int self_opp = (b * kQ + Opp(i)) * kNS + dst;
-              if (!s_in) {
-                srcf[e] = ReflectsOnPull(k) ? self_opp : e;
-                continue;
-              }
-              const bool s_core = in_core(sx - 1) && in_core(sy - 1) && in_core(sz - 1);
-              if (ReflectsOnPull(k) && !s_core) {
-                srcf[e] = self_opp;
-                continue;
-              }
-              const int sk = s_core ? kind(b, sx - 1, sy - 1, sz - 1) : kBulk;
-              if (sk == kSolid || sk == kBouzidi) {
-                const int64_t key = (static_cast<int64_t>(b) * kNC + (ix * kN + iy) * kN + iz) * kQ + i;
-                const auto it = qmap.find(key);
-                const double qf = it == qmap.end() ? 1.0 : it->second;
-                if (qf > 1.0e-10 && qf < 1.0 - 1.0e-10) {
-                  const int nx = hx + Cx(i), ny = hy + Cy(i), nz = hz + Cz(i);
-                  const int nk = (in_core(nx - 1) && in_core(ny - 1) && in_core(nz - 1))
-                                     ? kind(b, nx - 1, ny - 1, nz - 1)
-                                     : kBulk;
-                  AdjLink L{};
-                  L.row = e;
-                  L.bb = self_opp;
-                  L.upper = qf >= 0.5 - 1.0e-14;
-                  L.other = L.upper ? (nk == kBulk ? resolve(b, (nx * kNP + ny) * kNP + nz, i) : e) : e;
-                  L.q = qf;
-                  link_index[key] = static_cast<int>(links.size());
-                  srcf[e] = -1 - static_cast<int>(links.size());
-                  links.push_back(L);
-                  continue;
-                }
-                srcf[e] = self_opp;
-                continue;
-              }
-              srcf[e] = resolve(b, (sx * kNP + sy) * kNP + sz, i);
-            }
-          }
-      lv_link[lvl(b) + 1] = static_cast<int>(links.size());
-    }
-    for (int l = 1; l <= nlev; ++l) lv_link[l] = std::max(lv_link[l], lv_link[l - 1]);
-    nlinks = static_cast<int>(links.size());
-    // ---- live slots: the core and whatever the core's rows reach
-    std::vector<uint8_t> live(static_cast<size_t>(nb) * kNS, 0);
-    std::vector<int> work;
-    auto mark = [&](int e) {
-      const int b = e / (kQ * kNS), slot = e % kNS;
-      const size_t s = static_cast<size_t>(b) * kNS + slot;
-      if (!live[s]) {
-        live[s] = 1;
-        work.push_back(static_cast<int>(s));
+    // ---- live slots: the core (first, in (x, y, z) order), then the halo
+    // slots that the core's rows reach, ascending.  A halo slot is reached only
+    // from its own block (an exchanged one resolves to another block's core),
+    // so blocks are searched independently.
+    std::vector<short> rank(static_cast<size_t>(nb) * kNS, -1);
+    std::vector<uint8_t> plain(nb, 1);
+    std::vector<int> blinks(nb, 0);
+    block_cnt.assign(nb, 0);
+    ParallelFor(nb, [&](int b) {
+      short* rk = &rank[static_cast<size_t>(b) * kNS];
+      for (int c = 0; c < kNC && plain[b]; ++c) {
+        const int k = t.kinds[static_cast<size_t>(b) * kNC + c];
+        if (k == kSolid || ReflectsOnPull(k)) plain[b] = 0;
       }
-    };
-    for (int b = 0; b < nb; ++b)
-      for (int c = 0; c < kNC; ++c) {
-        const int ix = c / (kN * kN), iy = (c / kN) % kN, iz = c % kN;
-        mark((b * kQ) * kNS + ((ix + 1) * kNP + iy + 1) * kNP + iz + 1);
-      }
-    while (!work.empty()) {
-      const int s = work.back();
-      work.pop_back();
-      const int b = s / kNS, slot = s % kNS;
-      for (int i = 0; i < kQ; ++i) {
-        const int r = srcf[(static_cast<size_t>(b) * kQ + i) * kNS + slot];
-        if (r >= 0) {
-          mark(r);
-        } else {
-          mark(links[-1 - r].bb);
-          mark(links[-1 - r].other);
+      std::vector<int> work;
+      auto mark = [&](int sb, int slot) {
+        if (sb == b && rk[slot] < 0) {
+          rk[slot] = 0;
+          work.push_back(slot);
         }
+      };
+      for (int c = 0; c < kNC; ++c) rk[((c / (kN * kN) + 1) * kNP + c / kN % kN + 1) * kNP + c % kN + 1] = 0;
+      auto follow = [&](int slot) {
+        for (int i = 0; i < kQ; ++i) {
+          const Row r = row(b, plain[b], slot, i);
+          mark(r.b, r.slot);
+          if (r.link) {
+            mark(r.ob, r.oslot);
+            ++blinks[b];
+          }
+        }
+      };
+      for (int c = 0; c < kNC; ++c) {
+        const int ix = c / (kN * kN), iy = c / kN % kN, iz = c % kN;
+        const bool inner = ix > 0 && ix < kN - 1 && iy > 0 && iy < kN - 1 && iz > 0 && iz < kN - 1;
+        if (!(inner && plain[b])) follow(((ix + 1) * kNP + iy + 1) * kNP + iz + 1);
       }
-    }
-    // ---- compact numbering
-    std::vector<int> rank(static_cast<size_t>(nb) * kNS, -1), boff(nb), cnt(nb), first_cell(nb);
-    int total = 0;
-    cells.clear();
-    ckind.clear();
-    cell_block.clear();
-    cell_slot.clear();
-    core_cell.assign(static_cast<size_t>(nb) * kNC, -1);
+      while (!work.empty()) {
+        const int slot = work.back();
+        work.pop_back();
+        follow(slot);
+      }
+      int n = kNC;
+      for (int slot = 0; slot < kNS; ++slot) {
+        if (rk[slot] < 0) continue;
+        rk[slot] = static_cast<short>(
+            core_slot(slot) ? ((slot / (kNP * kNP) - 1) * kN + slot / kNP % kNP - 1) * kN + slot % kNP - 1 : n++);
+      }
+      block_cnt[b] = n;
+    });
+    // ---- numbering: blocks, levels and links in level order
+    std::vector<int> first_cell(nb), link_base(nb);
+    block_off.assign(nb, 0);
     lv_cell.assign(nlev + 1, 0);
     lv_entry.assign(nlev + 1, 0);
-    block_off.assign(nb, 0);
-    block_cnt.assign(nb, 0);
-    for (int bi = 0; bi < nb; ++bi) {
-      const int b = border[bi];
-      // core cells first in (x, y, z) order, then the live halo slots
-      std::vector<int> order;
-      for (int c = 0; c < kNC; ++c)
-        order.push_back(((c / (kN * kN) + 1) * kNP + (c / kN) % kN + 1) * kNP + c % kN + 1);
-      for (int slot = 0; slot < kNS; ++slot) {
-        const int px = slot / (kNP * kNP), py = (slot / kNP) % kNP, pz = slot % kNP;
-        if (live[static_cast<size_t>(b) * kNS + slot] && !(in_core(px - 1) && in_core(py - 1) && in_core(pz - 1)))
-          order.push_back(slot);
-      }
-      int r = 0;
-      for (int slot : order) rank[static_cast<size_t>(b) * kNS + slot] = r++;
-      cnt[b] = r;
-      boff[b] = total;
-      total += kQ * r;
-      first_cell[b] = static_cast<int>(cells.size());
-      for (int slot : order) {
-        const int rk = rank[static_cast<size_t>(b) * kNS + slot];
-        const int px = slot / (kNP * kNP), py = (slot / kNP) % kNP, pz = slot % kNP;
-        const bool core = in_core(px - 1) && in_core(py - 1) && in_core(pz - 1);
-        if (core) core_cell[static_cast<size_t>(b) * kNC + ((px - 1) * kN + py - 1) * kN + pz - 1] =
-            static_cast<int>(cells.size());
-        cells.push_back(Cell{boff[b] + rk, r});
-        ckind.push_back(core ? kind(b, px - 1, py - 1, pz - 1) : kHalo);
-        cell_block.push_back(b);
-        cell_slot.push_back(slot);
-      }
-      lv_cell[lvl(b) + 1] = static_cast<int>(cells.size());
-      lv_entry[lvl(b) + 1] = total;
-      block_off[b] = boff[b];
-      block_cnt[b] = r;
+    lv_link.assign(nlev + 1, 0);
+    ntot = ncells = nlinks = 0;
+    for (int b : border) {
+      block_off[b] = ntot;
+      first_cell[b] = ncells;
+      link_base[b] = nlinks;
+      ntot += kQ * block_cnt[b];
+      ncells += block_cnt[b];
+      nlinks += blinks[b];
+      lv_cell[lvl(b) + 1] = ncells;
+      lv_entry[lvl(b) + 1] = ntot;
+      lv_link[lvl(b) + 1] = nlinks;
     }
     for (int l = 1; l <= nlev; ++l) {
       lv_cell[l] = std::max(lv_cell[l], lv_cell[l - 1]);
       lv_entry[l] = std::max(lv_entry[l], lv_entry[l - 1]);
+      lv_link[l] = std::max(lv_link[l], lv_link[l - 1]);
     }
-    ntot = total;
-    ncells = static_cast<int>(cells.size());
-    auto cmap = [&](int e) {
-      const int b = e / (kQ * kNS), i = (e / kNS) % kQ, slot = e % kNS;
-      return boff[b] + i * cnt[b] + rank[static_cast<size_t>(b) * kNS + slot];
-    };
-    auto cell_of = [&](int e) {
-      const int b = e / (kQ * kNS), slot = e % kNS;
-      return first_cell[b] + rank[static_cast<size_t>(b) * kNS + slot];
-    };
-    std::vector<int> src(static_cast<size_t>(ntot), 0);
-    for (int b = 0; b < nb; ++b)
+    const std::vector<int>&boff = block_off, &cnt = block_cnt;
+    auto cmap = [&](int b, int slot, int i) { return boff[b] + i * cnt[b] + rank[static_cast<size_t>(b) * kNS + slot]; };
+    // ---- sources of every entry, and how often each is read (a copy counts 1,
+    // a Bouzidi row 65536)
+    cells.resize(ncells);
+    ckind.resize(ncells);
+    cell_block.resize(ncells);
+    cell_slot.resize(ncells);
+    core_cell.resize(static_cast<size_t>(nb) * kNC);
+    // big arrays are left to the threads to touch first: the kernel hands out
+    // pages at 2 GB/s to one thread
+    const size_t st = static_cast<size_t>(ntot);
+    const std::unique_ptr<int[]> src(new int[st]), rd(new int[st]);
+    const std::unique_ptr<uint32_t[]> nread(new uint32_t[st]);
+    ParallelFor(nb, [&](int b) {
+      std::fill_n(&nread[boff[b]], kQ * cnt[b], 0u);
+      std::fill_n(&rd[boff[b]], kQ * cnt[b], -1);
+    });
+    auto readers_of = [&](int e) { return static_cast<int>((nread[e] & 0xFFFF) + (nread[e] >> 16)); };
+    std::vector<AdjLink> links(nlinks);
+    std::vector<int64_t> link_key(nlinks);
+    auto read = [&](int e, int by) { __atomic_fetch_add(&nread[e], static_cast<uint32_t>(by), __ATOMIC_RELAXED); };
+    ParallelFor(nb, [&](int b) {
+      int lk = link_base[b];
       for (int slot = 0; slot < kNS; ++slot) {
-        if (rank[static_cast<size_t>(b) * kNS + slot] < 0) continue;
+        const int rk = rank[static_cast<size_t>(b) * kNS + slot];
+        if (rk < 0) continue;
+        const int cell = first_cell[b] + rk;
+        cells[cell] = Cell{boff[b] + rk, cnt[b]};
+        cell_block[cell] = b;
+        cell_slot[cell] = slot;
+        ckind[cell] = kHalo;
+        if (rk < kNC) {
+          core_cell[static_cast<size_t>(b) * kNC + rk] = cell;
+          ckind[cell] = t.kinds[static_cast<size_t>(b) * kNC + rk];
+        }
         for (int i = 0; i < kQ; ++i) {
-          const int e = (b * kQ + i) * kNS + slot;
-          src[cmap(e)] = srcf[e] >= 0 ? cmap(srcf[e]) : srcf[e];
+          const Row r = row(b, plain[b], slot, i);
+          const int e = cmap(b, slot, i), from = cmap(r.b, r.slot, r.pop);
+          if (!r.link) {
+            src[e] = from;
+            read(from, 1);
+            continue;
+          }
+          AdjLink L{};
+          L.row = e;
+          L.bb = from;
+          L.other = cmap(r.ob, r.oslot, i);
+          L.upper = r.upper;
+          L.q = r.q;
+          L.bb_cell = first_cell[r.b] + rank[static_cast<size_t>(r.b) * kNS + r.slot];
+          L.bb_pop = r.pop;
+          L.ot_cell = first_cell[r.ob] + rank[static_cast<size_t>(r.ob) * kNS + r.oslot];
+          L.ot_pop = i;
+          read(L.bb, 0x10000);
+          read(L.other, 0x10000);
+          link_key[lk] = r.key;
+          links[lk] = L;
+          src[e] = -1 - lk++;
         }
       }
-    for (AdjLink& L : links) {
-      L.bb_cell = cell_of(L.bb);
-      L.bb_pop = (L.bb / kNS) % kQ;
-      L.ot_cell = cell_of(L.other);
-      L.ot_pop = (L.other / kNS) % kQ;
-      L.row = cmap(L.row);
-      L.bb = cmap(L.bb);
-      L.other = cmap(L.other);
-    }
-    // ---- readers of every entry (the transpose of M)
-    std::vector<int> nread(static_cast<size_t>(ntot), 0), ncopy(static_cast<size_t>(ntot), 0);
-    for (int e = 0; e < ntot; ++e) {
-      if (src[e] >= 0) {
-        ++nread[src[e]];
-        ++ncopy[src[e]];
-      } else {
-        const AdjLink& L = links[-1 - src[e]];
-        ++nread[L.bb];
-        ++nread[L.other];
-      }
-    }
-    std::vector<int> rd(static_cast<size_t>(ntot), -1), ovo(1, 0), ovidx(static_cast<size_t>(ntot), -1);
-    for (int s = 0; s < ntot; ++s) {
-      if (nread[s] == 0) continue;
-      if (nread[s] == 1 && ncopy[s] == 1) continue;  // filled below
-      ovidx[s] = static_cast<int>(ovo.size()) - 1;
-      ovo.push_back(ovo.back() + nread[s]);
-      rd[s] = -2 - ovidx[s];
-    }
-    std::vector<int2> ove(static_cast<size_t>(ovo.back()));
-    std::vector<int> ofill(ovo.begin(), ovo.end() - 1);
-    for (int e = 0; e < ntot; ++e) {
-      if (src[e] >= 0) {
-        const int s = src[e];
-        if (ovidx[s] < 0) {
-          rd[s] = e;
+    });
+    for (int k = 0; k < nlinks; ++k) link_index[link_key[k]] = k;
+    // ---- readers of every entry (the transpose of M): the reader where it is
+    // one copy, else an overflow list in reader order
+    std::vector<int> nover(nb, 0), nove(nb, 0), none(nb, 0);
+    ParallelFor(nb, [&](int b) {
+      for (int e = boff[b]; e < boff[b] + kQ * cnt[b]; ++e)
+        if (nread[e] > 1) {
+          ++nover[b];
+          nove[b] += readers_of(e);
         } else {
-          ove[ofill[ovidx[s]]++] = make_int2(e, -1);
+          none[b] += nread[e] == 0;
         }
-      } else {
-        const int lk = -1 - src[e];
-        const AdjLink& L = links[lk];
-        ove[ofill[ovidx[L.bb]]++] = make_int2(e, 2 * lk);
-        ove[ofill[ovidx[L.other]]++] = make_int2(e, 2 * lk + 1);
-      }
+    });
+    std::vector<int> over_base(nb), ove_base(nb);
+    int over = 0, readers = 0;
+    int64_t counted = ntot;
+    for (int b : border) {
+      over_base[b] = over;
+      ove_base[b] = readers;
+      over += nover[b];
+      readers += nove[b];
+      counted += nove[b] - nover[b] - none[b];
     }
+    if (counted != static_cast<int64_t>(ntot) + nlinks) throw std::invalid_argument("adjoint: too many readers of an entry");
+    std::vector<int> ovo(static_cast<size_t>(over) + 1, readers), ofill(over);
+    std::vector<int2> ove(readers);
+    ParallelFor(nb, [&](int b) {
+      int o = over_base[b], at = ove_base[b];
+      for (int e = boff[b]; e < boff[b] + kQ * cnt[b]; ++e)
+        if (nread[e] > 1) {
+          rd[e] = -2 - o;
+          ofill[o] = ovo[o] = at;
+          ++o;
+          at += readers_of(e);
+        }
+    });
+    ParallelFor(nb, [&](int b) {
+      auto put = [&](int s, int e, int link) {
+        ove[__atomic_fetch_add(&ofill[-2 - rd[s]], 1, __ATOMIC_RELAXED)] = make_int2(e, link);
+      };
+      for (int e = boff[b]; e < boff[b] + kQ * cnt[b]; ++e) {
+        if (src[e] < 0) {
+          const int lk = -1 - src[e];
+          put(links[lk].bb, e, 2 * lk);
+          put(links[lk].other, e, 2 * lk + 1);
+        } else if (nread[src[e]] == 1) {
+          rd[src[e]] = e;
+        } else {
+          put(src[e], e, -1);
+        }
+      }
+    });
+    ParallelFor(nb, [&](int b) {
+      for (int o = over_base[b]; o < over_base[b] + nover[b]; ++o)
+        std::sort(ove.begin() + ovo[o], ove.begin() + ovo[o + 1],
+                  [](int2 p, int2 r) { return p.x != r.x ? p.x < r.x : p.y < r.y; });
+    });
     // ---- regular cells: entries computable from 27 neighbour-block bases
     nbase.assign(static_cast<size_t>(nb) * 27, make_int2(-1, 0));
-    for (int b = 0; b < nb; ++b) {
+    cblock.resize(ncells);
+    cflag.resize(ncells);
+    ParallelFor(nb, [&](int b) {
+      int2* nbb = &nbase[27 * static_cast<size_t>(b)];
       for (int o = 0; o < 27; ++o) {
         const int dx = o / 9 - 1, dy = (o / 3) % 3 - 1, dz = o % 3 - 1;
         if (dx == 0 && dy == 0 && dz == 0) {
-          nbase[27 * static_cast<size_t>(b) + o] = make_int2(boff[b], cnt[b]);
+          nbb[o] = make_int2(boff[b], cnt[b]);
           continue;
         }
         // the block that supplies this block's halo slot in that direction
         const int hx = dx < 0 ? 0 : (dx > 0 ? kNP - 1 : 1), hy = dy < 0 ? 0 : (dy > 0 ? kNP - 1 : 1),
                   hz = dz < 0 ? 0 : (dz > 0 ? kNP - 1 : 1);
         const int hs = t.halo_src[static_cast<size_t>(b) * kNS + (hx * kNP + hy) * kNP + hz];
-        if (hs < 0) continue;
-        nbase[27 * static_cast<size_t>(b) + o] = make_int2(boff[hs / kNS], cnt[hs / kNS]);
+        if (hs >= 0) nbb[o] = make_int2(boff[hs / kNS], cnt[hs / kNS]);
       }
-    }
-    auto regular_entry = [&](int b, int ix, int iy, int iz, int i) {
-      const int ox = ix < 0 ? 0 : (ix > kN - 1 ? 2 : 1), oy = iy < 0 ? 0 : (iy > kN - 1 ? 2 : 1),
-                oz = iz < 0 ? 0 : (iz > kN - 1 ? 2 : 1);
-      const int2 nbb = nbase[27 * static_cast<size_t>(b) + (ox * 3 + oy) * 3 + oz];
-      if (nbb.x < 0) return -1;
-      return nbb.x + i * nbb.y + (((ix & 7) * kN + (iy & 7)) * kN + (iz & 7));
-    };
-    cblock.assign(cells.size(), 0);
-    cflag.assign(cells.size(), 0);
-    for (size_t cl = 0; cl < cells.size(); ++cl) {
-      const int b = cell_block[cl];
-      cblock[cl] = b;
-      const int r = cells[cl].base - boff[b];
-      if (r >= kNC) continue;  // halo slot
-      const int ix = r >> 6, iy = (r >> 3) & 7, iz = r & 7;
-      bool fwd = true, rev = true;
-      for (int i = 0; i < kQ; ++i) {
-        const int e = cells[cl].base + i * cells[cl].stride;
-        const int fs = regular_entry(b, ix - Cx(i), iy - Cy(i), iz - Cz(i), i);
-        fwd = fwd && fs >= 0 && src[e] == fs;
-        const int rs = regular_entry(b, ix + Cx(i), iy + Cy(i), iz + Cz(i), i);
-        rev = rev && rs >= 0 && rd[e] == rs;
+      auto regular_entry = [&](int ix, int iy, int iz, int i) {
+        const int ox = ix < 0 ? 0 : (ix > kN - 1 ? 2 : 1), oy = iy < 0 ? 0 : (iy > kN - 1 ? 2 : 1),
+                  oz = iz < 0 ? 0 : (iz > kN - 1 ? 2 : 1);
+        const int2 v = nbb[(ox * 3 + oy) * 3 + oz];
+        if (v.x < 0) return -1;
+        return v.x + i * v.y + (((ix & 7) * kN + (iy & 7)) * kN + (iz & 7));
+      };
+      for (int r = 0; r < cnt[b]; ++r) {
+        const int cl = first_cell[b] + r;
+        cblock[cl] = b;
+        cflag[cl] = 0;
+        if (r >= kNC) continue;  // halo slot
+        const int ix = r >> 6, iy = (r >> 3) & 7, iz = r & 7;
+        bool fwd = true, rev = true;
+        for (int i = 0; i < kQ; ++i) {
+          const int e = cells[cl].base + i * cells[cl].stride;
+          const int fs = regular_entry(ix - Cx(i), iy - Cy(i), iz - Cz(i), i);
+          fwd = fwd && fs >= 0 && src[e] == fs;
+          const int rs = regular_entry(ix + Cx(i), iy + Cy(i), iz + Cz(i), i);
+          rev = rev && rs >= 0 && rd[e] == rs;
+        }
+        cflag[cl] = static_cast<uint8_t>((fwd ? 1 : 0) | (rev ? 2 : 0));
       }
-      cflag[cl] = static_cast<uint8_t>((fwd ? 1 : 0) | (rev ? 2 : 0));
-    }
+    });
     ADJ_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     d_cells = Alloc<Cell>(cells.size());
     d_cblock = Alloc<int>(cblock.size());
@@ -1087,13 +1149,12 @@ struct octlb_adj {
     ADJ_CHECK(hipMemcpy(d_cflag, cflag.data(), cflag.size(), hipMemcpyHostToDevice));
     ADJ_CHECK(hipMemcpy(d_nbase, nbase.data(), nbase.size() * sizeof(int2), hipMemcpyHostToDevice));
     d_ckind = Alloc<uint8_t>(ckind.size());
-    d_src = Alloc<int>(src.size());
-    d_rd = Alloc<int>(rd.size());
+    d_src = Alloc<int>(st);
+    d_rd = Alloc<int>(st);
     d_ovo = Alloc<int>(ovo.size());
     d_ove = Alloc<int2>(ove.size());
     d_links = Alloc<AdjLink>(links.size());
     d_dq = Alloc<double>(links.size());
-    const size_t st = static_cast<size_t>(ntot);
     d_y[0] = Alloc<unsigned char>(st * selem);
     d_y[1] = Alloc<unsigned char>(st * selem);
     d_lx = Alloc<double>(st);
@@ -1101,8 +1162,8 @@ struct octlb_adj {
     d_final = Alloc<unsigned char>(st * selem);
     ADJ_CHECK(hipMemcpy(d_cells, cells.data(), cells.size() * sizeof(Cell), hipMemcpyHostToDevice));
     ADJ_CHECK(hipMemcpy(d_ckind, ckind.data(), ckind.size(), hipMemcpyHostToDevice));
-    ADJ_CHECK(hipMemcpy(d_src, src.data(), src.size() * sizeof(int), hipMemcpyHostToDevice));
-    ADJ_CHECK(hipMemcpy(d_rd, rd.data(), rd.size() * sizeof(int), hipMemcpyHostToDevice));
+    ADJ_CHECK(hipMemcpy(d_src, src.get(), st * sizeof(int), hipMemcpyHostToDevice));
+    ADJ_CHECK(hipMemcpy(d_rd, rd.get(), st * sizeof(int), hipMemcpyHostToDevice));
     ADJ_CHECK(hipMemcpy(d_ovo, ovo.data(), ovo.size() * sizeof(int), hipMemcpyHostToDevice));
     if (!ove.empty()) ADJ_CHECK(hipMemcpy(d_ove, ove.data(), ove.size() * sizeof(int2), hipMemcpyHostToDevice));
     if (!links.empty())

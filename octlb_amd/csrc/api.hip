@@ -1722,6 +1722,35 @@ void CheckDev(const octlb_dev* d) {
   if (d == nullptr) throw ArgError("null device handle");
 }
 
+// Origins and, per halo slot, the block and slot that the exchange fills it from
+// (-1: none).  The part a slot belongs to is the same in every block.
+void ExportHalo(const octlb_dev* d, AdjTopo* t) {
+  constexpr int NP = kTile + 2, NS = NP * NP * NP;
+  BlockTab parts{};
+  for (int k = 0; k < 18; ++k) parts.nbr[k] = k;
+  struct Slot {
+    int slot, part, from;
+  };
+  std::vector<Slot> slots;
+  for (int s = 0; s < NS; ++s) {
+    const int x = s / (NP * NP) - 1, y = s / NP % NP - 1, z = s % NP - 1;
+    if (x >= 0 && x < kTile && y >= 0 && y < kTile && z >= 0 && z < kTile) continue;
+    int cc = 0;
+    const int part = ApronNeighbour(parts, x, y, z, &cc);
+    const int cx = cc / (kTile * kTile), cy = (cc / kTile) % kTile, cz = cc % kTile;
+    if (part >= 0) slots.push_back({s, part, ((cx + 1) * NP + cy + 1) * NP + cz + 1});
+  }
+  t->origin_cw.resize(static_cast<size_t>(d->nb) * 4);
+  t->halo_src.assign(static_cast<size_t>(d->nb) * NS, -1);
+  for (int b = 0; b < d->nb; ++b) {
+    const BlockTab& r = d->bt[b];
+    for (int a = 0; a < 3; ++a) t->origin_cw[4 * b + a] = r.origin[a];
+    t->origin_cw[4 * b + 3] = r.cw;
+    for (const Slot& s : slots)
+      if (r.nbr[s.part] >= 0) t->halo_src[static_cast<size_t>(b) * NS + s.slot] = r.nbr[s.part] * NS + s.from;
+  }
+}
+
 }  // namespace
 
 namespace octlb {
@@ -1737,7 +1766,6 @@ void ExportAdjTopo(const octlb_dev* d, AdjTopo* t) {
     throw std::invalid_argument("adjoint: needs the concrete handler, plain BGK and Bouzidi streaming");
   for (uint8_t k : d->kinds)
     if (IsFd(k)) throw std::invalid_argument("adjoint: FD boundary kinds are not differentiated");
-  constexpr int NP = kTile + 2, NS = NP * NP * NP;
   t->nb = d->nb;
   t->prec = d->prec;
   t->omega = d->sc.omega;
@@ -1748,26 +1776,7 @@ void ExportAdjTopo(const octlb_dev* d, AdjTopo* t) {
     t->link_key.push_back(kv.first);
     t->link_q.push_back(kv.second);
   }
-  t->origin_cw.resize(static_cast<size_t>(d->nb) * 4);
-  t->halo_src.assign(static_cast<size_t>(d->nb) * NS, -1);
-  for (int b = 0; b < d->nb; ++b) {
-    const BlockTab& r = d->bt[b];
-    for (int a = 0; a < 3; ++a) t->origin_cw[4 * b + a] = r.origin[a];
-    t->origin_cw[4 * b + 3] = r.cw;
-    for (int px = 0; px < NP; ++px)
-      for (int py = 0; py < NP; ++py)
-        for (int pz = 0; pz < NP; ++pz) {
-          const int x = px - 1, y = py - 1, z = pz - 1;
-          const bool core = x >= 0 && x < kTile && y >= 0 && y < kTile && z >= 0 && z < kTile;
-          if (core) continue;
-          int cc = 0;
-          const int nbk = ApronNeighbour(r, x, y, z, &cc);
-          if (nbk < 0) continue;
-          const int cx = cc / (kTile * kTile), cy = (cc / kTile) % kTile, cz = cc % kTile;
-          t->halo_src[static_cast<size_t>(b) * NS + (px * NP + py) * NP + pz] =
-              nbk * NS + ((cx + 1) * NP + cy + 1) * NP + cz + 1;
-        }
-  }
+  ExportHalo(d, t);
 }
 
 bool AdjNeedsMultiLevel(const octlb_dev* d) {
@@ -1787,7 +1796,6 @@ void ExportAdjMLTopo(octlb_dev* d, AdjTopo* t, AdjMLTopo* m) {
   if (d->nmembers != 1) throw std::invalid_argument("adjoint: ensembles are not differentiated");
   if (d->sc.handler != OCTLB_HANDLER_CONCRETE || d->sc.const_rho || !d->sc.bouzidi)
     throw std::invalid_argument("adjoint: needs the concrete handler, plain BGK and Bouzidi streaming");
-  constexpr int NP = kTile + 2, NS = NP * NP * NP;
   t->nb = d->nb;
   t->prec = d->prec;
   t->omega = d->sc.omega;
@@ -1798,25 +1806,7 @@ void ExportAdjMLTopo(octlb_dev* d, AdjTopo* t, AdjMLTopo* m) {
     t->link_key.push_back(kv.first);
     t->link_q.push_back(kv.second);
   }
-  t->origin_cw.resize(static_cast<size_t>(d->nb) * 4);
-  t->halo_src.assign(static_cast<size_t>(d->nb) * NS, -1);
-  for (int b = 0; b < d->nb; ++b) {
-    const BlockTab& r = d->bt[b];
-    for (int a = 0; a < 3; ++a) t->origin_cw[4 * b + a] = r.origin[a];
-    t->origin_cw[4 * b + 3] = r.cw;
-    for (int px = 0; px < NP; ++px)
-      for (int py = 0; py < NP; ++py)
-        for (int pz = 0; pz < NP; ++pz) {
-          const int x = px - 1, y = py - 1, z = pz - 1;
-          if (x >= 0 && x < kTile && y >= 0 && y < kTile && z >= 0 && z < kTile) continue;
-          int cc = 0;
-          const int nbk = ApronNeighbour(r, x, y, z, &cc);
-          if (nbk < 0) continue;
-          const int cx = cc / (kTile * kTile), cy = (cc / kTile) % kTile, cz = cc % kTile;
-          t->halo_src[static_cast<size_t>(b) * NS + (px * NP + py) * NP + pz] =
-              nbk * NS + ((cx + 1) * NP + cy + 1) * NP + cz + 1;
-        }
-  }
+  ExportHalo(d, t);
   t->level = d->level;
   m->max_level = d->max_level;
   m->level = d->level;
