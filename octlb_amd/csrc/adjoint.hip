@@ -18,14 +18,15 @@
 // block, its live slots in ascending slot order as population planes,
 //   state[block_offset + pop * live_slots(block) + rank(slot)]
 // so that threads over a block's cells read each plane coalesced.
-//   forward  KAdjCollide (first step of a sweep), then KAdjStep per step:
-//            gather x' = M y through one source index per entry (Bouzidi
-//            rows through a link record), store x', collide it into the
-//            next y (double-buffered)
-//   reverse  KAdjReverse per step: lambda_y = M^T lambda_x through one
-//            reader index per entry (the few entries read more than once
-//            or by a Bouzidi row go through an overflow list), then the BGK
-//            vector-Jacobian product at the stored pre-collide state;
+//   forward  KAdjCollide (first step of a sweep), then KAdjLinkRows and
+//            KAdjStep per step: gather x' = M y through one source index per
+//            entry (Bouzidi rows are formed first, behind y's entries), store
+//            x', collide it into the next y (double-buffered)
+//   reverse  KAdjReaders and KAdjReverse per step: lambda_y = M^T lambda_x
+//            through one reader index per entry (the few entries read more
+//            than once or by a Bouzidi row are summed first, behind lambda_x's
+//            entries), then the BGK vector-Jacobian product at the stored
+//            pre-collide state;
 //            the drag seeds of the step ride along; KAdjLinkGrad adds
 //            d out / d q on the Bouzidi rows (tiny)
 // The forward keeps a checkpoint every K steps; the reverse sweep recomputes
@@ -234,22 +235,24 @@ __device__ __forceinline__ int RegularEntry(const ADJ_RO int2* nbase, int ix, in
   return nb.x + i * nb.y + (((ix & 7) * kN + (iy & 7)) * kN + (iz & 7));
 }
 
-// entry e of x' = M y, rounded to the state's precision (Bouzidi rows are
-// evaluated in FP64 for every storage type, as the forward does)
-template <typename S, typename PY, typename PS, typename PL>
-__device__ __forceinline__ S RowValue(PY y, PS src, PL links, int e) {
-  const int s = src[e];
-  if (s >= 0) return y[s];
-  const AdjLink L = links[-1 - s];
+// Bouzidi rows [k0, k1) of x' = M y, appended to y as entries ntot + k, so that
+// streaming is one load per population for every cell; rounded to the state's
+// precision (the rows are evaluated in FP64 for every storage type, as the
+// forward does)
+template <typename S>
+__global__ __launch_bounds__(kThreads) void KAdjLinkRows(S* y, const AdjLink* links, int k0, int k1, int ntot) {
+  const int k = k0 + static_cast<int>(blockIdx.x) * kThreads + static_cast<int>(threadIdx.x);
+  if (k >= k1) return;
+  const AdjLink L = links[k];
   const double a = y[L.bb], o = y[L.other];
-  return static_cast<S>(L.upper ? BouzidiPull(a, o, o, L.q) : BouzidiPull(a, a, o, L.q));
+  y[ntot + k] = static_cast<S>(L.upper ? BouzidiPull(a, o, o, L.q) : BouzidiPull(a, a, o, L.q));
 }
 
 // x' = M y for this cell's entries, stored when x is given, then collided
 // into the next y
 template <typename S>
 __global__ __launch_bounds__(kThreads) void KAdjStep(const S* y, S* x, S* yn, const int* src,
-                                                     const AdjLink* links, const Cell* cells, const uint8_t* ckind,
+                                                     const Cell* cells, const uint8_t* ckind,
                                                      const int* cblock, const uint8_t* cflag, const int2* nbase,
                                                      int ncells, double omega) {
   const int t = XcdWg(blockIdx.x, gridDim.x) * kThreads + threadIdx.x;
@@ -269,7 +272,7 @@ __global__ __launch_bounds__(kThreads) void KAdjStep(const S* y, S* x, S* yn, co
 #pragma unroll
     for (int i = 0; i < kQ; ++i) {
       const int e = c.base + i * c.stride;
-      f[i] = RowValue<S>(Ro(y), Ro(src), Ro(links), e);
+      f[i] = Ro(y)[Ro(src)[e]];
       if (x) x[e] = f[i];
     }
   }
@@ -282,14 +285,13 @@ __global__ __launch_bounds__(kThreads) void KAdjStep(const S* y, S* x, S* yn, co
 // consecutive terms (tree order fixed), summed on the host in order; the
 // live value is the stream row of the post-collide state
 template <typename S>
-__global__ __launch_bounds__(kThreads) void KAdjDrag(const S* y, const int* src, const AdjLink* links,
-                                                     const DragTerm* terms, int nterms, double* out) {
+__global__ __launch_bounds__(kThreads) void KAdjDrag(const S* y, const int* src, const DragTerm* terms, int nterms, double* out) {
   __shared__ double red[kThreads];
   const int t = blockIdx.x * kThreads + threadIdx.x;
   double acc = 0.0;
   if (t < nterms) {
     const DragTerm d = terms[t];
-    acc = d.w * (static_cast<double>(y[d.snap]) + static_cast<double>(RowValue<S>(y, src, links, d.live)));
+    acc = d.w * (static_cast<double>(y[d.snap]) + static_cast<double>(y[src[d.live]]));
   }
   red[threadIdx.x] = acc;
   __syncthreads();
@@ -316,13 +318,30 @@ __device__ __forceinline__ double ReaderCoef(AdjLink L, int which) {
   return which ? 1.0 - 2.0 * L.q : 2.0 * L.q;
 }
 
+// M^T lx of the entries with several readers or a Bouzidi row (overflow lists
+// [o0, o1) of ovo / ove: row, -1 for a copy or 2 link + which), appended to lx as
+// entries ntot + o, a thread each.  Walked inside the reverse kernels instead, a
+// list is a chain of four dependent loads in front of the other populations.
+// Together with KAdjLinkRows this took the reverse sweep (with its recomputed
+// steps) of a 2-level cylinder channel from 267 to 219 ms (320 steps, FP32) and
+// that of a one-level box of 1M cells from 149 to 121 ms (400 steps, FP64).
+__global__ __launch_bounds__(kThreads) void KAdjReaders(double* lx, const int* ovo, const int2* ove,
+                                                        const AdjLink* links, int o0, int o1, int ntot) {
+  const int o = o0 + static_cast<int>(blockIdx.x) * kThreads + static_cast<int>(threadIdx.x);
+  if (o >= o1) return;
+  double v = 0.0;
+  for (int j = ovo[o]; j < ovo[o + 1]; ++j) {
+    const int2 r = ove[j];
+    v += (r.y < 0 ? 1.0 : ReaderCoef(links[r.y >> 1], r.y & 1)) * lx[r.x];
+  }
+  lx[ntot + o] = v;
+}
+
 // lxn = C^T (M^T lx) at the pre-collide state xp.  rd[e] >= 0: the one
-// output that copies e; -1: none; -2 - k: overflow list k (several readers
-// or a Bouzidi row) in ovo / ove (row, -1 for a copy or 2 link + which).
+// output that copies e, or its sum that KAdjReaders appended; -1: none.
 template <typename S>
 __global__ __launch_bounds__(kThreads) void KAdjReverse(const double* lx, double* lxn, const S* xp,
-                                                        const int* rd, const int* ovo, const int2* ove,
-                                                        const AdjLink* links, const Cell* cells,
+                                                        const int* rd, const Cell* cells,
                                                         const uint8_t* ckind, const int* cblock, const uint8_t* cflag,
                                                         const int2* nbase, const int* cseed, const double* seed_w,
                                                         double snap_scale, double live_scale, int ncells,
@@ -340,17 +359,7 @@ __global__ __launch_bounds__(kThreads) void KAdjReverse(const double* lx, double
 #pragma unroll
     for (int i = 0; i < kQ; ++i) {
       const int r = Ro(rd)[c.base + i * c.stride];
-      double v = 0.0;
-      if (r >= 0) {
-        v = Ro(lx)[r];
-      } else if (r < -1) {
-        const int k = -2 - r;
-        for (int j = Ro(ovo)[k]; j < Ro(ovo)[k + 1]; ++j) {
-          const int2 o = Ro(ove)[j];
-          v += (o.y < 0 ? 1.0 : ReaderCoef(Ro(links)[o.y >> 1], o.y & 1)) * Ro(lx)[o.x];
-        }
-      }
-      l[i] = v;
+      l[i] = r >= 0 ? Ro(lx)[r] : 0.0;
     }
   }
   // drag cells: the step's post-collide seed enters before the collide
@@ -487,15 +496,15 @@ __global__ __launch_bounds__(kThreads) void KMLCollide(const S* x, S* y, const C
 
 // x = M y over the entries of cells [c0, c1)
 template <typename S>
-__global__ __launch_bounds__(kThreads) void KMLGather(const S* y, S* x, const int* src, const AdjLink* links,
-                                                      const Cell* cells, int c0, int c1) {
+__global__ __launch_bounds__(kThreads) void KMLGather(const S* y, S* x, const int* src, const Cell* cells,
+                                                      int c0, int c1) {
   const int cl = c0 + static_cast<int>(blockIdx.x) * kThreads + static_cast<int>(threadIdx.x);
   if (cl >= c1) return;
   const Cell c = cells[cl];
 #pragma unroll
   for (int i = 0; i < kQ; ++i) {
     const int e = c.base + i * c.stride;
-    x[e] = RowValue<S>(y, src, links, e);
+    x[e] = y[src[e]];
   }
 }
 
@@ -547,7 +556,6 @@ __device__ inline void VelocityCollideVjp(const double* f, double* l, double ome
 // velocity cells as one partial per workgroup (fixed tree) in dui.
 template <typename S>
 __global__ __launch_bounds__(kThreads) void KMLVisitVjp(const double* lx, double* lxn, const S* xp, const int* rd,
-                                                        const int* ovo, const int2* ove, const AdjLink* links,
                                                         const Cell* cells, const uint8_t* ckind,
                                                         const SimConst* scp, const int* cseed, const double* seed_w,
                                                         double snap_scale, int c0, int c1) {
@@ -558,17 +566,7 @@ __global__ __launch_bounds__(kThreads) void KMLVisitVjp(const double* lx, double
 #pragma unroll
   for (int i = 0; i < kQ; ++i) {
     const int r = rd[c.base + i * c.stride];
-    double v = 0.0;
-    if (r >= 0) {
-      v = lx[r];
-    } else if (r < -1) {
-      const int k = -2 - r;
-      for (int j = ovo[k]; j < ovo[k + 1]; ++j) {
-        const int2 o = ove[j];
-        v += (o.y < 0 ? 1.0 : ReaderCoef(links[o.y >> 1], o.y & 1)) * lx[o.x];
-      }
-    }
-    l[i] = v;
+    l[i] = r >= 0 ? lx[r] : 0.0;
   }
   const int sk = cseed[cl];
   if (sk >= 0 && snap_scale != 0.0) {
@@ -736,7 +734,7 @@ struct octlb_adj {
   std::vector<double> origin_cw;
   std::unordered_map<int64_t, int> link_index;  // (block*512 + cell)*19 + pop -> Bouzidi row
   std::vector<int> border;                      // blocks in level order
-  std::vector<int> lv_cell, lv_entry, lv_link;  // per level: [begin, end) of cells, entries, links
+  std::vector<int> lv_cell, lv_entry, lv_link, lv_over;  // per level: [begin, end) of cells, entries, links, lists
   // multi-level: per operation, the window [win_lo, win_hi) of state entries
   // its adjoint reads, and the windows' offsets in a packed per-step tape
   std::vector<long long> win_lo, win_hi, win_off;
@@ -1037,7 +1035,7 @@ struct octlb_adj {
           read(L.other, 0x10000);
           link_key[lk] = r.key;
           links[lk] = L;
-          src[e] = -1 - lk++;
+          src[e] = ntot + lk++;
         }
       }
     });
@@ -1057,13 +1055,18 @@ struct octlb_adj {
     std::vector<int> over_base(nb), ove_base(nb);
     int over = 0, readers = 0;
     int64_t counted = ntot;
+    lv_over.assign(nlev + 1, 0);
     for (int b : border) {
       over_base[b] = over;
       ove_base[b] = readers;
       over += nover[b];
       readers += nove[b];
       counted += nove[b] - nover[b] - none[b];
+      lv_over[lvl(b) + 1] = over;
     }
+    for (int l = 1; l <= nlev; ++l) lv_over[l] = std::max(lv_over[l], lv_over[l - 1]);
+    if (static_cast<int64_t>(ntot) + std::max(over, nlinks) >= (1ll << 31))
+      throw std::invalid_argument("adjoint: too many blocks");
     if (counted != static_cast<int64_t>(ntot) + nlinks) throw std::invalid_argument("adjoint: too many readers of an entry");
     std::vector<int> ovo(static_cast<size_t>(over) + 1, readers), ofill(over);
     std::vector<int2> ove(readers);
@@ -1071,7 +1074,7 @@ struct octlb_adj {
       int o = over_base[b], at = ove_base[b];
       for (int e = boff[b]; e < boff[b] + kQ * cnt[b]; ++e)
         if (nread[e] > 1) {
-          rd[e] = -2 - o;
+          rd[e] = ntot + o;
           ofill[o] = ovo[o] = at;
           ++o;
           at += readers_of(e);
@@ -1079,11 +1082,11 @@ struct octlb_adj {
     });
     ParallelFor(nb, [&](int b) {
       auto put = [&](int s, int e, int link) {
-        ove[__atomic_fetch_add(&ofill[-2 - rd[s]], 1, __ATOMIC_RELAXED)] = make_int2(e, link);
+        ove[__atomic_fetch_add(&ofill[rd[s] - ntot], 1, __ATOMIC_RELAXED)] = make_int2(e, link);
       };
       for (int e = boff[b]; e < boff[b] + kQ * cnt[b]; ++e) {
-        if (src[e] < 0) {
-          const int lk = -1 - src[e];
+        if (src[e] >= ntot) {
+          const int lk = src[e] - ntot;
           put(links[lk].bb, e, 2 * lk);
           put(links[lk].other, e, 2 * lk + 1);
         } else if (nread[src[e]] == 1) {
@@ -1155,10 +1158,10 @@ struct octlb_adj {
     d_ove = Alloc<int2>(ove.size());
     d_links = Alloc<AdjLink>(links.size());
     d_dq = Alloc<double>(links.size());
-    d_y[0] = Alloc<unsigned char>(st * selem);
-    d_y[1] = Alloc<unsigned char>(st * selem);
-    d_lx = Alloc<double>(st);
-    d_ln = Alloc<double>(st);
+    d_y[0] = Alloc<unsigned char>((st + nlinks) * selem);
+    d_y[1] = Alloc<unsigned char>((st + nlinks) * selem);
+    d_lx = Alloc<double>(st + over);
+    d_ln = Alloc<double>(st + over);
     d_final = Alloc<unsigned char>(st * selem);
     ADJ_CHECK(hipMemcpy(d_cells, cells.data(), cells.size() * sizeof(Cell), hipMemcpyHostToDevice));
     ADJ_CHECK(hipMemcpy(d_ckind, ckind.data(), ckind.size(), hipMemcpyHostToDevice));
@@ -1409,6 +1412,16 @@ struct octlb_adj {
   // state that the operation's adjoint reads is copied there first, and for a
   // prolongation the prev macros into ptape
   template <typename S>
+  void LinkRows(S* y, int k0, int k1) {
+    if (k1 > k0)
+      hipLaunchKernelGGL(KAdjLinkRows<S>, dim3(Blocks(k1 - k0)), dim3(kThreads), 0, stream, y, d_links, k0, k1, ntot);
+  }
+  void Readers(int o0, int o1) {
+    if (o1 > o0)
+      hipLaunchKernelGGL(KAdjReaders, dim3(Blocks(o1 - o0)), dim3(kThreads), 0, stream, d_lx, d_ovo, d_ove, d_links, o0,
+                         o1, ntot);
+  }
+  template <typename S>
   void MLApply(size_t k, S* x, S* y, S* prev, double t, S* tape, S* ptape) {
     const size_t pm = static_cast<size_t>(npts) * kMacro;
     const int2 op = ops[k];
@@ -1423,8 +1436,9 @@ struct octlb_adj {
         if (c1 <= c0) break;
         hipLaunchKernelGGL(KMLCollide<S>, dim3(Blocks(c1 - c0)), dim3(kThreads), 0, stream, x, y, d_cells, d_ckind,
                            d_cblock, d_boff, d_ocw, d_scm, t, c0, c1, tape);
-        hipLaunchKernelGGL(KMLGather<S>, dim3(Blocks(c1 - c0)), dim3(kThreads), 0, stream, y, x, d_src, d_links,
-                           d_cells, c0, c1);
+        LinkRows(y, lv_link[l], lv_link[l + 1]);
+        hipLaunchKernelGGL(KMLGather<S>, dim3(Blocks(c1 - c0)), dim3(kThreads), 0, stream, y, x, d_src, d_cells,
+                           c0, c1);
         break;
       }
       case kOpFd:
@@ -1456,8 +1470,9 @@ struct octlb_adj {
         if (k1 > k0)
           hipLaunchKernelGGL(KMLLinkGrad<S>, dim3(Blocks(k1 - k0)), dim3(kThreads), 0, stream, d_lx, tape, d_cells,
                              d_ckind, d_cblock, d_boff, d_ocw, d_scm, t, d_links, k0, k1, d_dq);
+        Readers(lv_over[l], lv_over[l + 1]);
         hipLaunchKernelGGL(KMLVisitVjp<S>, dim3(Blocks(c1 - c0)), dim3(kThreads), 0, stream, d_lx, d_ln, tape, d_rd,
-                           d_ovo, d_ove, d_links, d_cells, d_ckind, d_scm, cseed, seed_w, snap_scale, c0, c1);
+                           d_cells, d_ckind, d_scm, cseed, seed_w, snap_scale, c0, c1);
         const int nv = lv_vcell[l + 1] - lv_vcell[l];
         if (nv > 0) {
           const unsigned nwg = Blocks(nv);
@@ -1542,7 +1557,7 @@ struct octlb_adj {
       const int ndg = std::max(1, static_cast<int>(Blocks(nterms)));
       double* d_jv = static_cast<double*>(alloc(static_cast<size_t>(steps + 1) * ndg * sizeof(double)));
       S* x = static_cast<S*>(alloc(st * sizeof(S)));
-      S* y = static_cast<S*>(alloc(st * sizeof(S)));
+      S* y = static_cast<S*>(alloc((st + nlinks) * sizeof(S)));
       S* pv = static_cast<S*>(alloc(pmn * sizeof(S)));
       S* ck = static_cast<S*>(alloc(static_cast<size_t>(nck) * st * sizeof(S)));
       S* ckp = static_cast<S*>(alloc(static_cast<size_t>(nck) * pmn * sizeof(S)));
@@ -1808,10 +1823,11 @@ struct octlb_adj {
                          ncells, omega);
       int cur = 0;
       for (int s = 1; s <= steps; ++s) {
+        LinkRows(ys[cur], 0, nlinks);
         hipLaunchKernelGGL(KAdjStep<S>, dim3(ncb), dim3(kThreads), 0, stream, ys[cur], xdest(s), ys[cur ^ 1], d_src,
-                           d_links, d_cells, d_ckind, d_cblock, d_cflag, d_nbase, ncells, omega);
+                           d_cells, d_ckind, d_cblock, d_cflag, d_nbase, ncells, omega);
         if (s > w0 && s <= w1 && nterms)
-          hipLaunchKernelGGL(KAdjDrag<S>, dim3(ndg), dim3(kThreads), 0, stream, ys[cur], d_src, d_links, d_terms, nterms,
+          hipLaunchKernelGGL(KAdjDrag<S>, dim3(ndg), dim3(kThreads), 0, stream, ys[cur], d_src, d_terms, nterms,
                              d_jv + static_cast<size_t>(s) * ndg);
         cur ^= 1;
       }
@@ -1832,8 +1848,9 @@ struct octlb_adj {
                              omega);
           int yc = 0;
           for (int j = 1; j < s1 - s0; ++j) {
+            LinkRows(ys[yc], 0, nlinks);
             hipLaunchKernelGGL(KAdjStep<S>, dim3(ncb), dim3(kThreads), 0, stream, ys[yc], xs(j), ys[yc ^ 1], d_src,
-                               d_links, d_cells, d_ckind, d_cblock, d_cflag, d_nbase, ncells, omega);
+                               d_cells, d_ckind, d_cblock, d_cflag, d_nbase, ncells, omega);
             yc ^= 1;
           }
         }
@@ -1843,8 +1860,9 @@ struct octlb_adj {
           if (nlinks)
             hipLaunchKernelGGL(KAdjLinkGrad<S>, dim3(Blocks(nlinks)), dim3(kThreads), 0, stream, d_lx, xp, d_cells,
                                d_ckind, d_links, nlinks, omega, d_dq);
-          hipLaunchKernelGGL(KAdjReverse<S>, dim3(ncb), dim3(kThreads), 0, stream, d_lx, d_ln, xp, d_rd, d_ovo, d_ove,
-                             d_links, d_cells, d_ckind, d_cblock, d_cflag, d_nbase, d_cseed, d_seed_w,
+          Readers(0, lv_over.back());
+          hipLaunchKernelGGL(KAdjReverse<S>, dim3(ncb), dim3(kThreads), 0, stream, d_lx, d_ln, xp, d_rd,
+                             d_cells, d_ckind, d_cblock, d_cflag, d_nbase, d_cseed, d_seed_w,
                              win(s) ? scale : 0.0, win(s - 1) ? scale : 0.0, ncells, omega);
           std::swap(d_lx, d_ln);
         }
