@@ -124,8 +124,8 @@ __device__ __forceinline__ T StreamPop(int i, const T* pl, const T* po, const ui
 // lane only picks among at most four uniform destinations by the sides it
 // crosses.  Looking the neighbour up by lane instead puts a vector load and a
 // wait for every store so far (loads and stores share a counter) before each
-// of the 18 stores: the fine level of the 2-level cylinder took 33.9 us in FP32
-// and 56.3 us in FP64 that way, 28.9 and 47.8 us this way.
+// of the 18 stores: the fine level of the 2-level cylinder took 32.9 us in FP32
+// and 55.6 us in FP64 that way, 26.9 and 47.8 us this way.
 template <typename T, bool kOwn>
 __device__ __forceinline__ void PushCell(const T* f, const OCTLB_CONST_TABLE BlockTab* bt, int b, int x, int y, int z,
                                          T* dst) {
