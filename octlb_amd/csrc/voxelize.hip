@@ -45,6 +45,7 @@
 #include <vector>
 
 #include "exact.h"
+#include "launch.h"
 #include "octlb_gpu.h"
 #include "octlb_internal.h"
 
@@ -241,6 +242,7 @@ struct VoxArgs {
   const double* bounds;
   int n;
   int te;               // tiles per block edge
+  int first;            // the launch's first tile (open_tiles entry)
   int channel;          // internal channel (else external obstacle)
   uint8_t* material;
   int* open_tiles;
@@ -284,7 +286,8 @@ __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
   __shared__ int nq, ng, open_here;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = a.n, tpb = a.te * a.te * a.te;
-  const int tile = kExact ? a.open_tiles[blockIdx.x] : static_cast<int>(blockIdx.x);
+  const int at = a.first + static_cast<int>(blockIdx.x);
+  const int tile = kExact ? a.open_tiles[at] : at;
   const int b = tile / tpb, tt = tile % tpb;
   // tiles in MaterialField order: x fastest
   const int org[3] = {tt % a.te * kVoxTile, tt / a.te % a.te * kVoxTile, tt / (a.te * a.te) * kVoxTile};
@@ -558,14 +561,19 @@ int VoxelizePart(int32_t num_blocks, int32_t n, const double* bounds, int64_t nu
   VOX_CHECK(hipMemcpy(buf.At<double>(o_bounds), bounds, static_cast<size_t>(num_blocks) * 6 * sizeof(double),
                       hipMemcpyHostToDevice));
   VOX_CHECK(hipMemset(a.open, 0, 2 * sizeof(unsigned int)));
-  hipLaunchKernelGGL(KClassify<false>, dim3(static_cast<unsigned>(ntile)), dim3(kVoxThreads), 0, nullptr, a);
-  VOX_CHECK(hipGetLastError());
+  // blocks of 9^3 or 10^3 cells have eight tiles, most of their cells idle:
+  // 1.6e9 cells are 17.6 million workgroups
+  auto classify = [&](auto kernel, int64_t tiles) {
+    ForLaunches(tiles, kVoxThreads, [&](int64_t first, int64_t count) {
+      a.first = static_cast<int>(first);
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(count)), dim3(kVoxThreads), 0, nullptr, a);
+      VOX_CHECK(hipGetLastError());
+    });
+  };
+  classify(KClassify<false>, ntile);
   unsigned int open[2] = {0, 0};
   VOX_CHECK(hipMemcpy(open, a.open, sizeof(open), hipMemcpyDeviceToHost));
-  if (open[1] > 0) {
-    hipLaunchKernelGGL(KClassify<true>, dim3(open[1]), dim3(kVoxThreads), 0, nullptr, a);
-    VOX_CHECK(hipGetLastError());
-  }
+  classify(KClassify<true>, open[1]);
   VOX_CHECK(hipMemcpy(material, a.material, total, hipMemcpyDeviceToHost));
   if (num_exact) *num_exact = open[0];
   return OCTLB_OK;
