@@ -48,6 +48,7 @@
 #include "launch.h"
 #include "octlb_gpu.h"
 #include "octlb_internal.h"
+#include "voxelize_queue.h"
 
 namespace octlb {
 namespace {
@@ -281,7 +282,7 @@ template <bool kExact>
 __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
   __shared__ uint32_t st[kVoxCells];
   __shared__ double cl[3][kVoxTile], ch[3][kVoxTile], cc[3][kVoxTile], inv[3];
-  __shared__ uint32_t queue[kVoxQueue];
+  __shared__ VoxEntry queue[kVoxQueue];
   __shared__ int groups[kVoxThreads];
   __shared__ int nq, ng, open_here;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -317,9 +318,8 @@ __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
 
   auto work = [&](int count) {
     for (int q = tid / kVoxLanes; q < count; q += kVoxThreads / kVoxLanes) {
-      const uint32_t e = queue[q];
-      const VTri& t = a.tris[e >> 2];
-      const int l = static_cast<int>(e & 3);
+      const VTri& t = a.tris[VoxTriangle(queue[q])];
+      const int l = VoxList(queue[q]);
       int lo[3], hi[3];  // the cells in reach, per axis
       if (l == 0) {
         for (int d = 0; d < 3; ++d) {
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
           for (int d = 0; d < 6; ++d) bx[d] = a.box[static_cast<size_t>(d) * a.ntri + t];
           const int in = Lists(bx, tb);
           for (int l = 0; l < 4; ++l)
-            if (in >> l & 1) queue[atomicAdd(&nq, 1)] = static_cast<uint32_t>(t) * 4u + l;
+            if (in >> l & 1) queue[atomicAdd(&nq, 1)] = MakeVoxEntry(t, l);
         }
       }
       __syncthreads();
