@@ -202,10 +202,26 @@ __global__ __launch_bounds__(kLinkThreads) void KGroupBox(const double* tris, in
   }
 }
 
+// No computed point of an edge inside the box (lo[3], hi[3]) is at a smaller
+// computed squared distance from p.  A point a + t (b - a), 0 <= t <= 1, may come
+// out up to 5 2^-53 M beyond the box along an axis, M the box's largest
+// coordinate there: 2 M for each rounding of b - a and of its product with t, M
+// for the sum.  So the gap gives way by 2^-50 M first, whatever its own size; the
+// relative roundings of p - q, the squares and the sum stay far below 1e-12.
+__device__ __forceinline__ double BoxDistance2(const double* bx, const double* p) {
+  double lb = 0.0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const double lo = bx[d], hi = bx[3 + d];
+    const double h = fmax(fmax(lo - p[d], p[d] - hi) - 0x1p-50 * fmax(fabs(lo), fabs(hi)), 0.0);
+    lb += h * h;
+  }
+  return lb * (1.0 - 1.0e-12);
+}
+
 // One wave per candidate cell: nearest soup point, then the 18 populations.
-// The search goes by groups: a group whose box is farther (squared distance,
-// lowered by 1e-12 relative -- far beyond its rounding error) than the best
-// point so far holds neither a closer nor an equal minimum, and the first
+// The search goes by groups: a group whose box is farther (BoxDistance2) than
+// the best point so far holds neither a closer nor an equal minimum, and the first
 // group searched is the nearest one, so few are left.  Testing every triangle's
 // box, staged in LDS 256 at a time with a barrier, took 257 us for 3,328 cells
 // and 8,192 triangles; by groups it is 17.9 us.
@@ -231,15 +247,11 @@ __global__ __launch_bounds__(kLinkThreads) void KNearest(const int2* cand, int64
   int64_t bt = INT64_MAX;
   double w[3] = {p[0], p[1], p[2]};
   const int64_t gs = GroupSize(ntri);
-  // squared distance of group g's box, lowered past its rounding error
   auto lower = [&](int64_t g) {
-    double lb = 0.0;
+    double bx[6];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const double h = fmax(fmax(gbox[d * ngroup + g] - p[d], p[d] - gbox[(3 + d) * ngroup + g]), 0.0);
-      lb += h * h;
-    }
-    return lb * (1.0 - 1.0e-12);
+    for (int d = 0; d < 6; ++d) bx[d] = gbox[d * ngroup + g];
+    return BoxDistance2(bx, p);
   };
   auto search = [&](int64_t g) {
     const int64_t t1 = ntri < (g + 1) * gs ? ntri : (g + 1) * gs;
