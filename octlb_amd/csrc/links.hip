@@ -52,6 +52,9 @@ __host__ __device__ inline int64_t GroupSize(int64_t ntri) {
   return 64 * ((ntri + 64 * kMaxGroups - 1) / (64 * kMaxGroups));
 }
 
+// Groups of a soup; none where a workgroup shares the whole soup in one go.
+int64_t GroupCount(int64_t ntri) { return ntri > kLinkThreads ? (ntri + GroupSize(ntri) - 1) / GroupSize(ntri) : 0; }
+
 __device__ __forceinline__ bool SolidLike(uint8_t m) { return m == 1 || m == 2; }  // kSolid, kBoundary
 
 // Material of cell (i, j, k) in MaterialField order (material_field.cpp:16-31).
@@ -173,7 +176,44 @@ __device__ __forceinline__ void TriClosest(const double* t, const double* p, dou
   }
 }
 
-// Bounding box (lo[3], hi[3]) of each group of consecutive triangles, one
+// A box (lo[3], hi[3]) that holds every computed point of the edges inside bx.  A
+// point a + t (b - a), 0 <= t <= 1, may come out up to 5 2^-53 M beyond the box
+// along an axis, M the box's largest coordinate there: 2 M for each rounding of
+// b - a and of its product with t, M for the sum.  Widened by 8 2^-53 M, less one
+// for this sum's own rounding.
+__device__ __forceinline__ void Widen(double* bx) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const double m = 0x1p-50 * fmax(fabs(bx[d]), fabs(bx[3 + d]));
+    bx[d] -= m;
+    bx[3 + d] += m;
+  }
+}
+
+// Widened box of a triangle.
+__device__ __forceinline__ void TriBox(const double* v, double* bx) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    bx[d] = fmin(v[d], fmin(v[3 + d], v[6 + d]));
+    bx[3 + d] = fmax(v[d], fmax(v[3 + d], v[6 + d]));
+  }
+  Widen(bx);
+}
+
+// No computed point of an edge inside the widened box bx is at a smaller computed
+// squared distance from p: the roundings of p - q, the squares and the sum stay far
+// below 1e-12 relative.
+__device__ __forceinline__ double BoxDistance2(const double* bx, const double* p) {
+  double lb = 0.0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const double h = fmax(fmax(bx[d] - p[d], p[d] - bx[3 + d]), 0.0);
+    lb += h * h;
+  }
+  return lb * (1.0 - 1.0e-12);
+}
+
+// Widened box (lo[3], hi[3]) of each group of consecutive triangles, one
 // array per bound; one wave per group.  A coordinate that is no number is left
 // out: the edges that hold it are at no distance from anything.
 __global__ __launch_bounds__(kLinkThreads) void KGroupBox(const double* tris, int64_t ntri, int64_t ngroup,
@@ -194,6 +234,7 @@ __global__ __launch_bounds__(kLinkThreads) void KGroupBox(const double* tris, in
       b[d] = fmin(b[d], __shfl_xor(b[d], w));
       b[3 + d] = fmax(b[3 + d], __shfl_xor(b[3 + d], w));
     }
+  Widen(b);
   if (lane < 6) {
     double out = b[0];
 #pragma unroll
@@ -202,37 +243,32 @@ __global__ __launch_bounds__(kLinkThreads) void KGroupBox(const double* tris, in
   }
 }
 
-// No computed point of an edge inside the box (lo[3], hi[3]) is at a smaller
-// computed squared distance from p.  A point a + t (b - a), 0 <= t <= 1, may come
-// out up to 5 2^-53 M beyond the box along an axis, M the box's largest
-// coordinate there: 2 M for each rounding of b - a and of its product with t, M
-// for the sum.  So the gap gives way by 2^-50 M first, whatever its own size; the
-// relative roundings of p - q, the squares and the sum stay far below 1e-12.
-__device__ __forceinline__ double BoxDistance2(const double* bx, const double* p) {
-  double lb = 0.0;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const double lo = bx[d], hi = bx[3 + d];
-    const double h = fmax(fmax(lo - p[d], p[d] - hi) - 0x1p-50 * fmax(fabs(lo), fabs(hi)), 0.0);
-    lb += h * h;
-  }
-  return lb * (1.0 - 1.0e-12);
-}
-
 // One wave per candidate cell: nearest soup point, then the 18 populations.
 // The search goes by groups: a group whose box is farther (BoxDistance2) than
 // the best point so far holds neither a closer nor an equal minimum, and the first
-// group searched is the nearest one, so few are left.  Testing every triangle's
-// box, staged in LDS 256 at a time with a barrier, took 257 us for 3,328 cells
-// and 8,192 triangles; by groups it is 17.9 us.
+// group searched is the nearest one, so few are left where consecutive triangles
+// near each other: 14.7 us for 3,328 cells and 8,192 triangles in the order of
+// their surface (257 us when every triangle's box was tested).
+//
+// Groups of triangles in any order, or of slivers across the domain, span it all
+// and none drops out.  Then a wave reads the whole soup, which L2 has to deliver
+// once per cell: the four waves of a workgroup share it instead, 256 triangles at a
+// time in LDS.  They do where three quarters of the groups hold the cell's centre,
+// or of a sample of the groups are left after the nearest one.  A sphere's
+// triangles shuffled, whole calls for 8,192 / 131,072 of them: 0.50 / 4.0 ms shared,
+// 0.80 / 9.0 ms each wave for itself (0.32 / 0.68 ms in surface order).
 // qd[cand][i-1] = q or -1; cnt[cand] = number of links of the cell.
 __global__ __launch_bounds__(kLinkThreads) void KNearest(const int2* cand, int64_t ncand, int n, const double* bounds,
                                                          const uint8_t* material, const double* tris, int64_t ntri,
                                                          const double* gbox, int64_t ngroup, double* qd, int* cnt) {
-  const int lane = threadIdx.x & 63;
-  const int64_t ci = static_cast<int64_t>(blockIdx.x) * (kLinkThreads / 64) + (threadIdx.x >> 6);
-  if (ci >= ncand) return;  // whole waves: no barrier below
-  const int2 ce = cand[ci];
+  constexpr int kWaves = kLinkThreads / 64;
+  __shared__ double staged[kLinkThreads * 9];
+  __shared__ double sbox[6][kLinkThreads];
+  __shared__ int left[kWaves];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t ci = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
+  const bool live = ci < ncand;  // waves without a cell only help to share triangles
+  const int2 ce = cand[live ? ci : ncand - 1];
   const int b = ce.x, c = ce.y;
   const int i = c / (n * n), j = (c / n) % n, k = c % n;
   const double* bb = bounds + 6 * static_cast<size_t>(b);
@@ -253,54 +289,112 @@ __global__ __launch_bounds__(kLinkThreads) void KNearest(const int2* cand, int64
     for (int d = 0; d < 6; ++d) bx[d] = gbox[d * ngroup + g];
     return BoxDistance2(bx, p);
   };
-  auto search = [&](int64_t g) {
-    const int64_t t1 = ntri < (g + 1) * gs ? ntri : (g + 1) * gs;
-    for (int64_t t = g * gs + lane; t < t1; t += 64) {
-      double v[9], q[3];
-#pragma unroll
-      for (int e = 0; e < 9; ++e) v[e] = tris[9 * t + e];
-      TriClosest(v, p, q);
-      const double d2 = (p[0] - q[0]) * (p[0] - q[0]) + (p[1] - q[1]) * (p[1] - q[1]) +
-                        (p[2] - q[2]) * (p[2] - q[2]);
-      if (d2 < bd || (d2 == bd && t < bt && bt != INT64_MAX)) {  // the first of equals
-        bd = d2;
-        bt = t;
-        w[0] = q[0];
-        w[1] = q[1];
-        w[2] = q[2];
-      }
-    }
+  // tests triangle t (v[9]); true where it is nearer than the wave's best
+  auto test = [&](const double* v, int64_t t) {
+    double q[3];
+    TriClosest(v, p, q);
+    const double d2 = (p[0] - q[0]) * (p[0] - q[0]) + (p[1] - q[1]) * (p[1] - q[1]) +
+                      (p[2] - q[2]) * (p[2] - q[2]);
+    if (!(d2 < bd || (d2 == bd && t < bt && bt != INT64_MAX))) return false;  // the first of equals
+    bd = d2;
+    bt = t;
+    w[0] = q[0];
+    w[1] = q[1];
+    w[2] = q[2];
+    return d2 < pb;
+  };
+  auto lower_best = [&]() {
     pb = bd;
     for (int off = 32; off > 0; off >>= 1) pb = fmin(pb, __shfl_xor(pb, off));
   };
-  double near = INFINITY;
-  int64_t first = 0;
-  for (int64_t g = lane; g < ngroup; g += 64) {
-    const double lb = lower(g);
-    if (lb < near) {
-      near = lb;
-      first = g;
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    const double od = __shfl_xor(near, off);
-    const int64_t og = __shfl_xor(first, off);
-    if (od < near || (od == near && og < first)) {
-      near = od;
-      first = og;
-    }
-  }
-  search(first);
-  for (int64_t g0 = 0; g0 < ngroup; g0 += 64) {
-    const int64_t g = g0 + lane;
-    uint64_t todo = __ballot(g < ngroup && g != first && !(lower(g < ngroup ? g : first) > pb));
+  // tests the groups whose bits are set from group g0 on; lb: the box distance of
+  // group g0 + lane, by which groups drop out as the best point gets nearer
+  auto search = [&](int64_t g0, uint64_t todo, double lb) {
     while (todo) {
-      const int at = __builtin_ctzll(todo);
+      const int64_t t0 = (g0 + __builtin_ctzll(todo)) * gs, t1 = ntri < t0 + gs ? ntri : t0 + gs;
       todo &= todo - 1;
-      search(g0 + at);
-      if (todo) todo &= __ballot(g < ngroup && !(lower(g < ngroup ? g : first) > pb));
+      bool nearer = false;
+      for (int64_t t = t0 + lane; t < t1; t += 64) {
+        double v[9], bx[6];
+#pragma unroll
+        for (int e = 0; e < 9; ++e) v[e] = tris[9 * t + e];
+        TriBox(v, bx);
+        if (!(BoxDistance2(bx, p) > fmin(bd, pb))) nearer = test(v, t) || nearer;
+      }
+      if (__any(nearer)) {
+        lower_best();
+        todo &= __ballot(!(lb > pb));
+      }
+    }
+  };
+  int64_t first = -1;  // the group searched first
+  int kept = 64;       // of 64 groups, how many are still to be searched
+  if (ngroup > 0) {
+    double near = INFINITY;
+    int64_t inside = 0;  // groups whose box holds p, which never drop out
+    for (int64_t g0 = 0; g0 < ngroup; g0 += 64) {
+      const int64_t g = g0 + lane;
+      const double lb = g < ngroup ? lower(g) : INFINITY;
+      inside += __popcll(__ballot(lb == 0.0));
+      if (lb < near) {
+        near = lb;
+        first = g;
+      }
+    }
+    if (4 * inside > 3 * ngroup) {
+      first = -1;
+    } else {
+      if (first < 0) first = 0;
+      for (int off = 32; off > 0; off >>= 1) {
+        const double od = __shfl_xor(near, off);
+        const int64_t og = __shfl_xor(first, off);
+        if (od < near || (od == near && og < first)) {
+          near = od;
+          first = og;
+        }
+      }
+      search(first, 1, 0.0);
+      kept = ngroup > 8 ? __popcll(__ballot(!(lower(lane * ngroup / 64) > pb))) : 0;
     }
   }
+  bool share = ngroup == 0;
+  if (!share) {
+    if (lane == 0) left[wave] = live ? kept : 0;
+    __syncthreads();
+    int sum = 0;
+    for (int k = 0; k < kWaves; ++k) sum += left[k];
+    share = sum > 48 * static_cast<int>(ncand - (ci - wave) < kWaves ? ncand - (ci - wave) : kWaves);
+  }
+  if (share) {
+    for (int64_t base = 0; base < ntri; base += kLinkThreads) {
+      const int nt = static_cast<int>(ntri - base < kLinkThreads ? ntri - base : kLinkThreads);
+      __syncthreads();  // the triangles before are no longer read
+      for (int e = threadIdx.x; e < 9 * nt; e += kLinkThreads) staged[e] = tris[9 * base + e];
+      if (static_cast<int>(threadIdx.x) < nt) {
+        double bx[6];
+        TriBox(tris + 9 * (base + threadIdx.x), bx);
+#pragma unroll
+        for (int d = 0; d < 6; ++d) sbox[d][threadIdx.x] = bx[d];
+      }
+      __syncthreads();
+      bool nearer = false;
+      for (int r = lane; r < nt; r += 64) {
+        double bx[6];
+#pragma unroll
+        for (int d = 0; d < 6; ++d) bx[d] = sbox[d][r];
+        if (!(BoxDistance2(bx, p) > fmin(bd, pb))) nearer = test(staged + 9 * r, base + r) || nearer;
+      }
+      if (__any(nearer)) lower_best();
+    }
+  } else if (live) {
+    for (int64_t g0 = 0; g0 < ngroup; g0 += 64) {
+      const int64_t g = g0 + lane;
+      const double lb = lower(g < ngroup ? g : 0);
+      const uint64_t todo = __ballot(g < ngroup && g != first && !(lb > pb));
+      if (todo) search(g0, todo, lb);
+    }
+  }
+  if (!live) return;
   // smallest distance over the wave, ties to the lowest triangle index
   for (int off = 32; off > 0; off >>= 1) {
     const double od = __shfl_xor(bd, off);
@@ -360,6 +454,13 @@ __global__ __launch_bounds__(kLinkThreads) void KEmit(const int2* cand, int64_t 
   q[at] = v;
 }
 
+void GroupBoxes(const double* tris, int64_t ntri, int64_t ngroup, double* gbox, hipStream_t s) {
+  if (ngroup == 0) return;
+  constexpr int kWaves = kLinkThreads / 64;
+  KGroupBox<<<static_cast<unsigned>((ngroup + kWaves - 1) / kWaves), kLinkThreads, 0, s>>>(tris, ntri, ngroup, gbox);
+  LINK_CHECK(hipGetLastError());
+}
+
 struct DevBuf {
   std::vector<void*> ptrs;
   template <typename P>
@@ -406,13 +507,11 @@ void BuildLinks(int32_t nb, int32_t n, const double* bounds, const uint8_t* mate
   LINK_CHECK(hipMemcpyAsync(&ncand, d_boff + nb, sizeof(int64_t), hipMemcpyDeviceToHost, st.s));
   LINK_CHECK(hipStreamSynchronize(st.s));
   if (ncand == 0) return;
-  int2* d_cand = mem.Get<int2>(ncand);
+  const int64_t ngroup = GroupCount(ntri);
+  double* d_gbox = mem.Get<double>(6 * static_cast<size_t>(ngroup) + ncand);  // and the candidates
+  int2* d_cand = reinterpret_cast<int2*>(d_gbox + 6 * ngroup);
+  GroupBoxes(d_tris, ntri, ngroup, d_gbox, st.s);
   KCandidates<true><<<nb, kLinkThreads, 0, st.s>>>(n, d_mat, nullptr, d_boff, d_cand);
-  LINK_CHECK(hipGetLastError());
-  const int64_t ngroup = (ntri + GroupSize(ntri) - 1) / GroupSize(ntri);
-  double* d_gbox = mem.Get<double>(6 * static_cast<size_t>(ngroup));
-  KGroupBox<<<static_cast<unsigned>((ngroup + kLinkThreads / 64 - 1) / (kLinkThreads / 64)), kLinkThreads, 0, st.s>>>(
-      d_tris, ntri, ngroup, d_gbox);
   LINK_CHECK(hipGetLastError());
   double* d_qd = mem.Get<double>(static_cast<size_t>(ncand) * (kQ - 1));
   int* d_cnt = mem.Get<int>(ncand);
@@ -510,11 +609,9 @@ void BuildLinksNoAlloc(int32_t nb, int32_t n, const double* d_bounds, const uint
   LINK_CHECK(hipGetLastError());
   const int64_t waves_per_wg = kLinkThreads / 64;
   const unsigned grid = static_cast<unsigned>((ncand + waves_per_wg - 1) / waves_per_wg);
-  const int64_t ngroup = (ntri + GroupSize(ntri) - 1) / GroupSize(ntri);
+  const int64_t ngroup = GroupCount(ntri);
   double* d_gbox = reinterpret_cast<double*>(base + kScrGbox);
-  KGroupBox<<<static_cast<unsigned>((ngroup + waves_per_wg - 1) / waves_per_wg), kLinkThreads, 0, s>>>(d_tris, ntri,
-                                                                                                      ngroup, d_gbox);
-  LINK_CHECK(hipGetLastError());
+  GroupBoxes(d_tris, ntri, ngroup, d_gbox, s);
   KNearest<<<grid, kLinkThreads, 0, s>>>(d_cand, ncand, n, d_bounds, d_mat, d_tris, ntri, d_gbox, ngroup, d_qd, d_cnt);
   LINK_CHECK(hipGetLastError());
   KScan<<<1, 1024, 0, s>>>(d_cnt, ncand, d_loff);
