@@ -191,10 +191,11 @@ struct octlb_dev {
   std::vector<int> member_begin;  // [nmembers + 1] block offsets
   std::vector<SimConst> scm;      // constants per member
   SimConst* d_scm = nullptr;
-  int* d_stat_tiles = nullptr;    // [nmembers + 1] stats-level tile offsets per member
-  int4* d_stat_chunk = nullptr;   // chunks of the reference-order sum (StatChunks)
+  int4* d_stat_chunk = nullptr;   // chunks of the average's sum (StatChunks)
   int* d_stat_chunk_begin = nullptr;  // [nmembers + 1]
   StatPart* d_stat_part = nullptr;
+  double2* d_stat_sum = nullptr;
+  unsigned int* d_stat_done = nullptr;  // [nmembers]
   int stat_chunks = 0;
   int* d_step = nullptr;   // [2]: double-buffered coarse-step counter
   int step_slot = 0;       // slot holding the current step's time
@@ -1098,16 +1099,19 @@ void octlb_dev::Prepare() {
     }
     if (!padded)
       for (int& t : tiles_of) t *= kTile;  // a partial per x plane
-    d_stat_tiles = PAlloc<int>(nmembers + 1);
-    Upload(d_stat_tiles, tiles_of, stream);
     std::vector<int> chunk_begin;
-    const std::vector<int4> chunk = StatChunks(cells, &chunk_begin);
+    const std::vector<int4> chunk = StatChunks(fast_stats ? tiles_of : cells, &chunk_begin);
     stat_chunks = static_cast<int>(chunk.size());
     d_stat_chunk = PAlloc<int4>(chunk.size());
     Upload(d_stat_chunk, chunk, stream);
     d_stat_chunk_begin = PAlloc<int>(chunk_begin.size());
     Upload(d_stat_chunk_begin, chunk_begin, stream);
     d_stat_part = PAlloc<StatPart>(chunk.size());
+    d_stat_sum = PAlloc<double2>(chunk.size());
+    const std::vector<unsigned int> zero(nmembers, 0u);
+    d_stat_done = PAlloc<unsigned int>(zero.size());
+    Upload(d_stat_done, zero, stream);
+    Sync();  // the tables above leave scope
   }
   Upload(d_bt, bt, stream);
   Sync();
@@ -1373,7 +1377,9 @@ void octlb_dev::Level(int l) {
       tile_updates += static_cast<double>(level_blocks[l]) * static_cast<double>(ncore);
     }
     par[l] ^= 1;
-    if (a.want_stats == 1) LaunchStatsFinalize<T>(d_stats, d_stat_tiles, nmembers, d_avg, stream);
+    if (a.want_stats == 1)
+      LaunchStatsFinalize(d_stats, d_stat_chunk, d_stat_chunk_begin, stat_chunks, d_stat_sum, d_stat_done, d_avg,
+                          stream);
     if (a.want_stats == 2)
       LaunchStatsSequential(d_stat_val, d_stat_use, d_stat_chunk, d_stat_chunk_begin, stat_chunks, nmembers,
                             d_stat_part, d_avg, stream);

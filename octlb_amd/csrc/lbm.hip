@@ -590,30 +590,71 @@ __global__ __launch_bounds__(512) void KPadded(TileArgs<T> a) {
 }
 
 // ------------------------------------------------------------ small kernels
-// Tree reduction of the per-tile partial sums (fast_stats: not the
-// reference's summation order, but a fixed one): one workgroup per member,
-// threads take strided tiles in order, then a pairwise reduction.
-constexpr int kStatsThreads = 256;
-__global__ __launch_bounds__(kStatsThreads) void KStatsFinalize(const double* partial, const int* tile_begin,
-                                                                double* avg) {
-  __shared__ double rs[kStatsThreads], rc[kStatsThreads];
-  const int m = blockIdx.x, tid = threadIdx.x;
-  double s = 0.0, c = 0.0;
-  for (int i = tile_begin[m] + tid; i < tile_begin[m + 1]; i += kStatsThreads) {
-    s += partial[2 * i];
-    c += partial[2 * i + 1];
+constexpr int kStatChunk = 1024;  // cells (ordered sum) or partials (fast) per chunk
+constexpr int kStatChunkThreads = 256;
+
+// Sum of a workgroup's (s, c) in a fixed order, in thread 0.
+__device__ inline void GroupSum(double& s, double& c, double* rs, double* rc) {
+  for (int w = 32; w > 0; w >>= 1) {
+    s += __shfl_down(s, w);
+    c += __shfl_down(c, w);
   }
-  rs[tid] = s;
-  rc[tid] = c;
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    rs[wave] = s;
+    rc[wave] = c;
+  }
   __syncthreads();
-  for (int w = kStatsThreads / 2; w > 0; w >>= 1) {
-    if (tid < w) {
-      rs[tid] += rs[tid + w];
-      rc[tid] += rc[tid + w];
+  if (threadIdx.x == 0)
+    for (int k = 1; k < kStatChunkThreads / 64; ++k) {
+      s += rs[k];
+      c += rc[k];
+    }
+  __syncthreads();  // rs, rc may be written again
+}
+
+// Tree reduction of the partial sums (fast_stats: not the reference's
+// summation order, but a fixed one): a workgroup per chunk of a member's
+// partials, the last of a member to finish (a device-scope counter, reset by it)
+// sums the chunks.  There is a partial for every 64 cells, and one workgroup
+// per member was bound by its own loads: a step of 224^3 cells took 927 us that
+// way and takes 647 us (FP32).
+__global__ __launch_bounds__(kStatChunkThreads) void KStatsFinalize(const double2* partial, const int4* chunk,
+                                                                    const int* chunk_begin, double2* sums,
+                                                                    unsigned int* done, double* avg) {
+  __shared__ double rs[kStatChunkThreads / 64], rc[kStatChunkThreads / 64];
+  __shared__ int last;
+  const int4 ch = chunk[blockIdx.x];  // first partial, end, member
+  const int m = ch.z, tid = threadIdx.x;
+  const int cb = chunk_begin[m], nc = chunk_begin[m + 1] - cb;
+  double s = 0.0, c = 0.0;
+#pragma unroll
+  for (int k = 0; k < kStatChunk / kStatChunkThreads; ++k) {
+    const int i = ch.x + k * kStatChunkThreads + tid;
+    if (i < ch.y) {
+      s += partial[i].x;
+      c += partial[i].y;
+    }
+  }
+  GroupSum(s, c, rs, rc);
+  if (nc > 1) {
+    if (tid == 0) {
+      sums[blockIdx.x] = make_double2(s, c);
+      __threadfence();  // the chunk's sum before the count that publishes it
+      last = atomicAdd(&done[m], 1u) == static_cast<unsigned int>(nc - 1);
     }
     __syncthreads();
+    if (!last) return;
+    __threadfence();  // every chunk's sum is visible to the last workgroup
+    s = c = 0.0;
+    for (int k = tid; k < nc; k += kStatChunkThreads) {
+      s += sums[cb + k].x;
+      c += sums[cb + k].y;
+    }
+    GroupSum(s, c, rs, rc);
+    if (tid == 0) done[m] = 0u;
   }
-  if (tid == 0) avg[m] = rc[0] > 0.0 ? rs[0] / rc[0] : 1.0;  // CollideRhoStats::average (block_lattice.h:31)
+  if (tid == 0) avg[m] = c > 0.0 ? s / c : 1.0;  // CollideRhoStats::average (block_lattice.h:31)
 }
 
 // CollideRhoStats accumulated in the reference's cell order (blocks of the
@@ -631,8 +672,6 @@ __global__ __launch_bounds__(kStatsThreads) void KStatsFinalize(const double* pa
 // predicts; KStatsWalk takes the chunks in order and adds one by one those whose
 // E was not the running sum's, that leave the binade, or that hold a value the
 // maps do not cover (negative, not finite, 2^E or more).
-constexpr int kStatChunk = 1024;       // cells per chunk
-constexpr int kStatChunkThreads = 256;
 constexpr int kStatBad = -100000;      // StatPart::e of a chunk without a usable pair
 
 __device__ inline StatPair Then(StatPair a, StatPair b) {
@@ -1869,17 +1908,18 @@ void LaunchTile(const TileArgs<T>& a, hipStream_t s) {
 
 static inline dim3 Grid(long long n, int bs) { return dim3(static_cast<unsigned>((n + bs - 1) / bs)); }
 
-template <typename T>
-void LaunchStatsFinalize(const double* partial, const int* tile_begin, int members, double* avg, hipStream_t s) {
-  hipLaunchKernelGGL(KStatsFinalize, dim3(members), dim3(kStatsThreads), 0, s, partial, tile_begin, avg);
+void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, double2* sums,
+                         unsigned int* done, double* avg, hipStream_t s) {
+  hipLaunchKernelGGL(KStatsFinalize, dim3(nchunk), dim3(kStatChunkThreads), 0, s,
+                     reinterpret_cast<const double2*>(partial), chunk, chunk_begin, sums, done, avg);
 }
 
-std::vector<int4> StatChunks(const std::vector<int>& cell_begin, std::vector<int>* chunk_begin) {
+std::vector<int4> StatChunks(const std::vector<int>& begin, std::vector<int>* chunk_begin) {
   std::vector<int4> chunk;
   chunk_begin->assign(1, 0);
-  for (size_t m = 0; m + 1 < cell_begin.size(); ++m) {
-    for (int k = cell_begin[m]; k < cell_begin[m + 1]; k += kStatChunk)
-      chunk.push_back(make_int4(k, std::min(k + kStatChunk, cell_begin[m + 1]), static_cast<int>(m), k - cell_begin[m]));
+  for (size_t m = 0; m + 1 < begin.size(); ++m) {
+    for (int k = begin[m]; k < begin[m + 1]; k += kStatChunk)
+      chunk.push_back(make_int4(k, std::min(k + kStatChunk, begin[m + 1]), static_cast<int>(m), k - begin[m]));
     chunk_begin->push_back(static_cast<int>(chunk.size()));
   }
   return chunk;
@@ -2036,7 +2076,6 @@ void LaunchMacro(const T* p0, const T* p1, const ParArray& par, const BlockTab* 
 
 #define OCTLB_INSTANTIATE(T)                                                                      \
   template void LaunchTile<T>(const TileArgs<T>&, hipStream_t);                                   \
-  template void LaunchStatsFinalize<T>(const double*, const int*, int, double*, hipStream_t);     \
   template void LaunchInitEq<T>(T*, const uint8_t*, int, const SimConst&, double, const double*,  \
                                 uint32_t, hipStream_t);                                           \
   template void LaunchInitField<T>(T*, int, const SimConst&, const double*, const double*,        \

@@ -487,13 +487,13 @@ __device__ __forceinline__ void CollideCell(T* f, int k, const SimConst& sc, con
 // --------------------------------------------------------------- launchers
 template <typename T>
 void LaunchTile(const TileArgs<T>& a, hipStream_t s);
-// ConstRho averages of the members: member m owns tiles [tile_begin[m],
-// tile_begin[m+1]) of the partial sums.
-template <typename T>
-void LaunchStatsFinalize(const double* partial, const int* tile_begin, int members, double* avg, hipStream_t s);
-// The reference-order sum goes by chunks of consecutive cells: (first cell,
-// end, member, cells of the member before it), member m owning chunks
-// [chunk_begin[m], chunk_begin[m + 1]); part holds one entry per chunk.
+// ConstRho averages of the members.  Both sums go by chunks of a member's
+// partials (fast) or cells (reference order): (first, end, member, how many of
+// the member's before it), member m owning begin[m] .. begin[m + 1] and chunks
+// [chunk_begin[m], chunk_begin[m + 1]); sums and part hold one entry per chunk,
+// done one zero per member.
+void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, double2* sums,
+                         unsigned int* done, double* avg, hipStream_t s);
 struct StatPair {
   long long d0, d1;  // what the chunk adds to an even / odd integer sum
 };
@@ -502,7 +502,7 @@ struct StatPart {
   int count;
   int e;  // exponent of the running sum the pair holds for
 };
-std::vector<int4> StatChunks(const std::vector<int>& cell_begin, std::vector<int>* chunk_begin);
+std::vector<int4> StatChunks(const std::vector<int>& begin, std::vector<int>* chunk_begin);
 void LaunchStatsSequential(const double* val, const uint8_t* use, const int4* chunk, const int* chunk_begin,
                            int nchunk, int members, StatPart* part, double* avg, hipStream_t s);
 void LaunchStepInc(const int* step, int* step_next, hipStream_t s);

@@ -1,0 +1,47 @@
+"""The ConstRho average summed by chunks of 1,024 partials (fast_stats), a
+partial per x plane of a block: members of less than a chunk, just below and
+above one, several; step by step and from a captured graph, against the average
+in the reference's order.  N positive values summed in any order are within
+(N - 1) 2^-53 of the exact sum, so the two differ by at most twice that, once per
+step taken."""
+import numpy as np
+import pytest
+
+from octlb_amd import cases
+from octlb_amd.solver import GpuSolver
+
+pytestmark = pytest.mark.gpu
+
+
+def _solver(sizes, precision, fast):
+    members = [cases.cavity_blocked(n, 0.6 + 0.05 * m, 0.03 + 0.01 * m, 1, x0=2.0 * m) for m, n in enumerate(sizes)]
+    ens = cases.ensemble(members, fast_stats=fast)
+    s = GpuSolver.ensemble(ens, precision)
+    s.set_bc_kinds(ens.kinds)
+    s.init_equilibrium(1.0, (0.0, 0.0, 0.0), 0xFF)
+    return s
+
+
+# 8 partials, 1,000 and 1,728 (a chunk is 1,024), 4 chunks; members of both kinds
+@pytest.mark.parametrize("sizes", [(8,), (40,), (48,), (64,), (48, 8, 40, 56)])
+@pytest.mark.parametrize("precision", [64, 32])
+def test_matches_the_ordered_average(sizes, precision):
+    fast, ordered = _solver(sizes, precision, 1), _solver(sizes, precision, 0)
+    for k, steps in enumerate((1, 1, 1, 4)):
+        for s in (fast, ordered):
+            if steps == 1:
+                s.advance(1)
+            else:
+                s.advance_graph(steps)
+        taken = 1 + k if steps == 1 else 3 + steps
+        for m, n in enumerate(sizes):
+            want = ordered.member_average_rho(m)
+            tol = 2 * taken * n ** 3 * 2.0 ** -53 if precision == 64 else 2 * taken * n ** 3 * 2.0 ** -53 + 2.0 ** -24
+            assert abs(fast.member_average_rho(m) - want) <= tol * want
+    again = _solver(sizes, precision, 1)
+    again.advance(3)
+    again.advance_graph(4)
+    assert [again.member_average_rho(m) for m in range(len(sizes))] == [fast.member_average_rho(m)
+                                                                       for m in range(len(sizes))]
+    for s in (fast, ordered, again):
+        s.close()
