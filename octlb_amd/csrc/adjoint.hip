@@ -38,17 +38,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstring>
-#include <exception>
 #include <functional>
 #include <memory>
-#include <mutex>
 #include <stdexcept>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -57,6 +52,7 @@
 #include "octlb_internal.h"
 #include "adjoint_ml.h"
 #include "adjoint_topo.h"
+#include "parallel_for.h"
 
 namespace octlb {
 namespace {
@@ -91,36 +87,6 @@ __device__ __forceinline__ int XcdWg(int w, int n) {
 constexpr int kN = 8, kNP = 10, kNS = kNP * kNP * kNP, kNC = kN * kN * kN;
 constexpr int kThreads = 128;
 constexpr uint8_t kHalo = 255;  // kind of a halo slot: carried, never collided
-
-// body(k) for k in [0, count), spread over the host's threads (at most 16);
-// what a body throws is thrown here.
-template <typename F>
-void ParallelFor(int count, F&& body) {
-  constexpr int kChunk = 16;
-  const int want = std::min({16, static_cast<int>(std::thread::hardware_concurrency()), count / kChunk});
-  std::atomic<int> next{0};
-  std::exception_ptr failed;
-  std::mutex failed_mu;
-  auto run = [&] {
-    try {
-      for (int k0; (k0 = next.fetch_add(kChunk)) < count;)
-        for (int k = k0; k < std::min(k0 + kChunk, count); ++k) body(k);
-    } catch (...) {
-      std::lock_guard<std::mutex> lock(failed_mu);
-      if (!failed) failed = std::current_exception();
-      next = count;
-    }
-  };
-  std::vector<std::thread> threads;
-  try {
-    while (static_cast<int>(threads.size()) + 1 < want) threads.emplace_back(run);
-  } catch (const std::system_error&) {
-    // fewer threads than wanted: those there are, and this one, do the work
-  }
-  run();
-  for (std::thread& th : threads) th.join();
-  if (failed) std::rethrow_exception(failed);
-}
 
 struct AdjLink {
   int row;      // output entry
