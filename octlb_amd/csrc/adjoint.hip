@@ -821,17 +821,10 @@ struct octlb_adj {
       *sb = hs >= 0 ? hs / kNS : b;
       *ss = hs >= 0 ? hs % kNS : slot;
     };
-    auto row = [&](int b, bool plain, int slot, int i) {
+    auto wall_row = [&](int b, int slot, int i) {  // of a core cell
       Row r{b, slot, i, false, false, 0, 0, 0, 0.0};
       const int off = (Cx(i) * kNP + Cy(i)) * kNP + Cz(i);
       const int hx = slot / (kNP * kNP), hy = slot / kNP % kNP, hz = slot % kNP;
-      const bool core = in_core(hx - 1) && in_core(hy - 1) && in_core(hz - 1);
-      if (!core || plain) {
-        // a core cell's source is never beyond the halo; a halo slot's wraps
-        const int s = slot - off;
-        resolve(b, s < 0 ? s + kNS : (s >= kNS ? s - kNS : s), &r.b, &r.slot);
-        return r;
-      }
       const int k = kind(b, hx - 1, hy - 1, hz - 1);
       if (k == kSolid) return r;
       const int sx = hx - Cx(i) - 1, sy = hy - Cy(i) - 1, sz = hz - Cz(i) - 1;
@@ -862,6 +855,34 @@ struct octlb_adj {
       resolve(b, slot - off, &r.b, &r.slot);
       return r;
     };
+    // Most rows are plain: the source is the slot against the velocity, or the
+    // core slot that the exchange fills it from.  Exceptions are core cells that
+    // are walls (of any kind) or stream from a solid one, told by a block's slots:
+    // 0 for fluid and halo, 1 for velocity and pressure, 2 for solid and Bouzidi.
+    std::vector<uint8_t> core(kNS);
+    for (int slot = 0; slot < kNS; ++slot) core[slot] = core_slot(slot);
+    int pull[kQ];
+    for (int i = 0; i < kQ; ++i) pull[i] = (Cx(i) * kNP + Cy(i)) * kNP + Cz(i);
+    struct Walls {
+      uint8_t at[kNS];
+      bool any;
+    };
+    auto find_walls = [&](int b, Walls* w) {
+      *w = {};
+      for (int c = 0; c < kNC; ++c) {
+        const int k = t.kinds[static_cast<size_t>(b) * kNC + c];
+        const uint8_t v = k == kSolid || k == kBouzidi ? 2 : (ReflectsOnPull(k) ? 1 : 0);
+        w->at[((c / (kN * kN) + 1) * kNP + c / kN % kN + 1) * kNP + c % kN + 1] = v;
+        w->any = w->any || v != 0;
+      }
+    };
+    // the slot that a plain row pulls from, -1 for another row.  A core cell's
+    // source is never beyond the halo; a halo slot's wraps.
+    auto plain_source = [&](const Walls& w, int slot, int i) {
+      const int s = slot - pull[i];
+      if (core[slot]) return w.at[slot] != 0 || w.at[s] == 2 ? -1 : s;
+      return s < 0 ? s + kNS : (s >= kNS ? s - kNS : s);
+    };
     // blocks in level order (a stable sort: one level keeps the block order),
     // so that every level's cells, entries and links are contiguous ranges
     border.resize(nb);
@@ -875,18 +896,17 @@ struct octlb_adj {
     // from its own block (an exchanged one resolves to another block's core),
     // so blocks are searched independently.
     std::vector<short> rank(static_cast<size_t>(nb) * kNS, -1);
-    std::vector<uint8_t> plain(nb, 1);
     std::vector<int> blinks(nb, 0);
     block_cnt.assign(nb, 0);
-    ParallelFor(nb, [&](int b) {
+    ParallelFor(nb, 1, [&](int b) {
       short* rk = &rank[static_cast<size_t>(b) * kNS];
-      for (int c = 0; c < kNC && plain[b]; ++c) {
-        const int k = t.kinds[static_cast<size_t>(b) * kNC + c];
-        if (k == kSolid || ReflectsOnPull(k)) plain[b] = 0;
-      }
+      const int* halo = &t.halo_src[static_cast<size_t>(b) * kNS];
+      Walls w;
+      find_walls(b, &w);
+      int found = 0;
       std::vector<int> work;
-      auto mark = [&](int sb, int slot) {
-        if (sb == b && rk[slot] < 0) {
+      auto mark = [&](int slot) {
+        if (rk[slot] < 0) {
           rk[slot] = 0;
           work.push_back(slot);
         }
@@ -894,18 +914,23 @@ struct octlb_adj {
       for (int c = 0; c < kNC; ++c) rk[((c / (kN * kN) + 1) * kNP + c / kN % kN + 1) * kNP + c % kN + 1] = 0;
       auto follow = [&](int slot) {
         for (int i = 0; i < kQ; ++i) {
-          const Row r = row(b, plain[b], slot, i);
-          mark(r.b, r.slot);
+          const int s = plain_source(w, slot, i);
+          if (s >= 0) {
+            if (halo[s] < 0) mark(s);
+            continue;
+          }
+          const Row r = wall_row(b, slot, i);
+          if (r.b == b) mark(r.slot);
           if (r.link) {
-            mark(r.ob, r.oslot);
-            ++blinks[b];
+            if (r.ob == b) mark(r.oslot);
+            ++found;
           }
         }
       };
       for (int c = 0; c < kNC; ++c) {
         const int ix = c / (kN * kN), iy = c / kN % kN, iz = c % kN;
         const bool inner = ix > 0 && ix < kN - 1 && iy > 0 && iy < kN - 1 && iz > 0 && iz < kN - 1;
-        if (!(inner && plain[b])) follow(((ix + 1) * kNP + iy + 1) * kNP + iz + 1);
+        if (!inner || w.any) follow(((ix + 1) * kNP + iy + 1) * kNP + iz + 1);
       }
       while (!work.empty()) {
         const int slot = work.back();
@@ -916,9 +941,10 @@ struct octlb_adj {
       for (int slot = 0; slot < kNS; ++slot) {
         if (rk[slot] < 0) continue;
         rk[slot] = static_cast<short>(
-            core_slot(slot) ? ((slot / (kNP * kNP) - 1) * kN + slot / kNP % kNP - 1) * kN + slot % kNP - 1 : n++);
+            core[slot] ? ((slot / (kNP * kNP) - 1) * kN + slot / kNP % kNP - 1) * kN + slot % kNP - 1 : n++);
       }
       block_cnt[b] = n;
+      blinks[b] = found;
     });
     // ---- numbering: blocks, levels and links in level order
     std::vector<int> first_cell(nb), link_base(nb);
@@ -957,18 +983,29 @@ struct octlb_adj {
     const size_t st = static_cast<size_t>(ntot);
     const std::unique_ptr<int[]> src(new int[st]), rd(new int[st]);
     const std::unique_ptr<uint32_t[]> nread(new uint32_t[st]);
-    ParallelFor(nb, [&](int b) {
+    ParallelFor(nb, 16, [&](int b) {
       std::fill_n(&nread[boff[b]], kQ * cnt[b], 0u);
       std::fill_n(&rd[boff[b]], kQ * cnt[b], -1);
     });
     auto readers_of = [&](int e) { return static_cast<int>((nread[e] & 0xFFFF) + (nread[e] >> 16)); };
     std::vector<AdjLink> links(nlinks);
     std::vector<int64_t> link_key(nlinks);
-    auto read = [&](int e, int by) { __atomic_fetch_add(&nread[e], static_cast<uint32_t>(by), __ATOMIC_RELAXED); };
-    ParallelFor(nb, [&](int b) {
+    // *at += by, by several threads unless alone (an atomic add takes 5 ns)
+    auto add = [](auto* at, auto by, bool alone) {
+      if (!alone) return __atomic_fetch_add(at, by, __ATOMIC_RELAXED);
+      const auto was = *at;
+      *at += by;
+      return was;
+    };
+    auto read = [&, alone = ParallelThreads(nb, 1) == 1](int e, uint32_t by) { add(&nread[e], by, alone); };
+    ParallelFor(nb, 1, [&](int b) {
+      const short* rks = &rank[static_cast<size_t>(b) * kNS];
+      const int* halo = &t.halo_src[static_cast<size_t>(b) * kNS];
+      Walls w;
+      find_walls(b, &w);
       int lk = link_base[b];
       for (int slot = 0; slot < kNS; ++slot) {
-        const int rk = rank[static_cast<size_t>(b) * kNS + slot];
+        const int rk = rks[slot];
         if (rk < 0) continue;
         const int cell = first_cell[b] + rk;
         cells[cell] = Cell{boff[b] + rk, cnt[b]};
@@ -980,8 +1017,16 @@ struct octlb_adj {
           ckind[cell] = t.kinds[static_cast<size_t>(b) * kNC + rk];
         }
         for (int i = 0; i < kQ; ++i) {
-          const Row r = row(b, plain[b], slot, i);
-          const int e = cmap(b, slot, i), from = cmap(r.b, r.slot, r.pop);
+          const int e = boff[b] + i * cnt[b] + rk;
+          const int s = plain_source(w, slot, i);
+          if (s >= 0) {
+            const int hs = halo[s];
+            src[e] = hs >= 0 ? boff[hs / kNS] + i * cnt[hs / kNS] + rank[hs] : boff[b] + i * cnt[b] + rks[s];
+            read(src[e], 1);
+            continue;
+          }
+          const Row r = wall_row(b, slot, i);
+          const int from = cmap(r.b, r.slot, r.pop);
           if (!r.link) {
             src[e] = from;
             read(from, 1);
@@ -1009,14 +1054,18 @@ struct octlb_adj {
     // ---- readers of every entry (the transpose of M): the reader where it is
     // one copy, else an overflow list in reader order
     std::vector<int> nover(nb, 0), nove(nb, 0), none(nb, 0);
-    ParallelFor(nb, [&](int b) {
+    ParallelFor(nb, 8, [&](int b) {
+      int lists = 0, entries = 0, unread = 0;  // the blocks' counts share cache lines
       for (int e = boff[b]; e < boff[b] + kQ * cnt[b]; ++e)
         if (nread[e] > 1) {
-          ++nover[b];
-          nove[b] += readers_of(e);
+          ++lists;
+          entries += readers_of(e);
         } else {
-          none[b] += nread[e] == 0;
+          unread += nread[e] == 0;
         }
+      nover[b] = lists;
+      nove[b] = entries;
+      none[b] = unread;
     });
     std::vector<int> over_base(nb), ove_base(nb);
     int over = 0, readers = 0;
@@ -1036,7 +1085,7 @@ struct octlb_adj {
     if (counted != static_cast<int64_t>(ntot) + nlinks) throw std::invalid_argument("adjoint: too many readers of an entry");
     std::vector<int> ovo(static_cast<size_t>(over) + 1, readers), ofill(over);
     std::vector<int2> ove(readers);
-    ParallelFor(nb, [&](int b) {
+    ParallelFor(nb, 16, [&](int b) {
       int o = over_base[b], at = ove_base[b];
       for (int e = boff[b]; e < boff[b] + kQ * cnt[b]; ++e)
         if (nread[e] > 1) {
@@ -1046,9 +1095,9 @@ struct octlb_adj {
           at += readers_of(e);
         }
     });
-    ParallelFor(nb, [&](int b) {
-      auto put = [&](int s, int e, int link) {
-        ove[__atomic_fetch_add(&ofill[rd[s] - ntot], 1, __ATOMIC_RELAXED)] = make_int2(e, link);
+    ParallelFor(nb, 4, [&](int b) {
+      auto put = [&, alone = ParallelThreads(nb, 4) == 1](int s, int e, int link) {
+        ove[add(&ofill[rd[s] - ntot], 1, alone)] = make_int2(e, link);
       };
       for (int e = boff[b]; e < boff[b] + kQ * cnt[b]; ++e) {
         if (src[e] >= ntot) {
@@ -1062,7 +1111,7 @@ struct octlb_adj {
         }
       }
     });
-    ParallelFor(nb, [&](int b) {
+    ParallelFor(nb, 16, [&](int b) {
       for (int o = over_base[b]; o < over_base[b] + nover[b]; ++o)
         std::sort(ove.begin() + ovo[o], ove.begin() + ovo[o + 1],
                   [](int2 p, int2 r) { return p.x != r.x ? p.x < r.x : p.y < r.y; });
@@ -1071,7 +1120,7 @@ struct octlb_adj {
     nbase.assign(static_cast<size_t>(nb) * 27, make_int2(-1, 0));
     cblock.resize(ncells);
     cflag.resize(ncells);
-    ParallelFor(nb, [&](int b) {
+    ParallelFor(nb, 2, [&](int b) {
       int2* nbb = &nbase[27 * static_cast<size_t>(b)];
       for (int o = 0; o < 27; ++o) {
         const int dx = o / 9 - 1, dy = (o / 3) % 3 - 1, dz = o % 3 - 1;
@@ -1098,12 +1147,14 @@ struct octlb_adj {
         cflag[cl] = 0;
         if (r >= kNC) continue;  // halo slot
         const int ix = r >> 6, iy = (r >> 3) & 7, iz = r & 7;
+        const bool inner = ix > 0 && ix < kN - 1 && iy > 0 && iy < kN - 1 && iz > 0 && iz < kN - 1;
         bool fwd = true, rev = true;
         for (int i = 0; i < kQ; ++i) {
           const int e = cells[cl].base + i * cells[cl].stride;
-          const int fs = regular_entry(ix - Cx(i), iy - Cy(i), iz - Cz(i), i);
+          const int step = (Cx(i) * kN + Cy(i)) * kN + Cz(i);
+          const int fs = inner ? e - step : regular_entry(ix - Cx(i), iy - Cy(i), iz - Cz(i), i);
+          const int rs = inner ? e + step : regular_entry(ix + Cx(i), iy + Cy(i), iz + Cz(i), i);
           fwd = fwd && fs >= 0 && src[e] == fs;
-          const int rs = regular_entry(ix + Cx(i), iy + Cy(i), iz + Cz(i), i);
           rev = rev && rs >= 0 && rd[e] == rs;
         }
         cflag[cl] = static_cast<uint8_t>((fwd ? 1 : 0) | (rev ? 2 : 0));

@@ -10,19 +10,26 @@
 
 namespace octlb {
 
-// body(k) for k in [0, count), spread over the host's threads (at most 16);
-// what a body throws is thrown here.
+// Threads that ParallelFor takes for `count` bodies, this one among them: one for
+// every `each` bodies beyond the first, at most 16.
+inline int ParallelThreads(int count, int each) {
+  return std::max(1, std::min({16, static_cast<int>(std::thread::hardware_concurrency()), 1 + (count - 1) / each}));
+}
+
+// body(k) for k in [0, count), spread over the host's threads; what a body throws
+// is thrown here.  `each`: bodies that are worth a thread, which takes about 25 us
+// to start.
 template <typename F>
-void ParallelFor(int count, F&& body) {
-  constexpr int kChunk = 16;
-  const int want = std::min({16, static_cast<int>(std::thread::hardware_concurrency()), count / kChunk});
+void ParallelFor(int count, int each, F&& body) {
+  const int want = ParallelThreads(count, each);
+  const int chunk = std::max(1, std::min(16, count / (8 * want)));
   std::atomic<int> next{0};
   std::exception_ptr failed;
   std::mutex failed_mu;
   auto run = [&] {
     try {
-      for (int k0; (k0 = next.fetch_add(kChunk)) < count;)
-        for (int k = k0; k < std::min(k0 + kChunk, count); ++k) body(k);
+      for (int k0; (k0 = next.fetch_add(chunk)) < count;)
+        for (int k = k0; k < std::min(k0 + chunk, count); ++k) body(k);
     } catch (...) {
       std::lock_guard<std::mutex> lock(failed_mu);
       if (!failed) failed = std::current_exception();
@@ -31,7 +38,7 @@ void ParallelFor(int count, F&& body) {
   };
   std::vector<std::thread> threads;
   try {
-    threads.reserve(want > 1 ? want - 1 : 0);
+    threads.reserve(want - 1);
     while (static_cast<int>(threads.size()) + 1 < want) threads.emplace_back(run);
   } catch (...) {
     // no memory or no thread for more: those there are, and this one, do the

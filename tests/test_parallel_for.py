@@ -31,9 +31,9 @@ void operator delete(void* p, std::size_t) noexcept { std::free(p); }
 
 static std::atomic<int> done[5000];
 
-static bool EveryIndexOnce(int count) {
+static bool EveryIndexOnce(int count, int each) {
   for (auto& d : done) d = 0;
-  octlb::ParallelFor(count, [](int k) { ++done[k]; });
+  octlb::ParallelFor(count, each, [](int k) { ++done[k]; });
   for (int k = 0; k < 5000; ++k)
     if (done[k] != (k < count ? 1 : 0)) return false;
   return true;
@@ -41,14 +41,15 @@ static bool EveryIndexOnce(int count) {
 
 int main() {
   for (int count : {0, 1, 2, 3, 15, 16, 17, 31, 32, 33, 256, 1000, 4097})
-    if (!EveryIndexOnce(count)) {
-      std::printf("count %d\n", count);
-      return 1;
-    }
+    for (int each : {1, 2, 16})
+      if (!EveryIndexOnce(count, each)) {
+        std::printf("count %d each %d\n", count, each);
+        return 1;
+      }
   for (int bad : {0, 17, 999}) {
     bool thrown = false;
     try {
-      octlb::ParallelFor(1000, [&](int k) {
+      octlb::ParallelFor(1000, 1, [&](int k) {
         if (k == bad) throw std::invalid_argument("body");
       });
     } catch (const std::invalid_argument&) {
@@ -61,7 +62,7 @@ int main() {
   }
   for (long k = 0; k < 24; ++k) {
     fail_at = allocations + k;
-    const bool good = EveryIndexOnce(4097);
+    const bool good = EveryIndexOnce(4097, 1);
     fail_at = -1;
     if (!good) {
       std::printf("allocation %ld\n", k);
