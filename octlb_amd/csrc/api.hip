@@ -599,8 +599,10 @@ void octlb_dev::Build(const octlb_topology* t, const octlb_params* p) {
   HIP_CHECK(hipMemsetAsync(d_kind, 0, kinds.size(), stream));
   d_bt = Alloc<BlockTab>(nb);
   Upload(d_bt, bt, stream);
-  d_tiles = Alloc<Tile>(tiles.size());
-  Upload(d_tiles, tiles, stream);
+  if (padded) {  // other forests' tiles depend on the cell kinds
+    d_tiles = Alloc<Tile>(tiles.size());
+    Upload(d_tiles, tiles, stream);
+  }
   {
     std::vector<int> rank(nb, 0), next(kMaxLevels, 0);
     for (int bi = 0; bi < nb; ++bi) rank[block_order[bi]] = next[level[block_order[bi]]]++;
@@ -830,6 +832,7 @@ void octlb_dev::Prepare() {
   // eight: 23,456 wall blocks of an ensemble took 926 us that way and 756 us
   // as pull tiles (FP32).
   npush_blocks = 0;
+  std::vector<int> push_blocks;
   if (!padded) {
     std::vector<char> is_push(nb, 0);
     for (int b = 0; b < nb; ++b) {
@@ -868,7 +871,6 @@ void octlb_dev::Prepare() {
     // time: with the push tasks in a launch of their own, which needs no LDS,
     // the 64-member ensemble took 1355 us a step where this order takes 1270
     // (FP32), the 2-level cylinder's finest level 52.8 against 47.8 (FP64).
-    std::vector<int> push_blocks;
     tiles.clear();
     for (int l = 0; l <= max_level; ++l) {
       tile_begin[l] = static_cast<int>(tiles.size());
@@ -897,7 +899,6 @@ void octlb_dev::Prepare() {
     Upload(d_tiles, tiles, stream);
     d_push_blocks = PAlloc<int>(push_blocks.size());
     Upload(d_push_blocks, push_blocks, stream);
-    Sync();  // the tables above leave scope
   }
   // ---- post-stream FD cell lists (concrete handler, tree-boundary blocks)
   std::vector<int2> fd_cells[3];
@@ -1068,6 +1069,9 @@ void octlb_dev::Prepare() {
   HIP_CHECK(hipMemsetAsync(d_drag_done, 0, sizeof(unsigned int), stream));
   // ConstRho statistics of the finest level, per member: the member's
   // tiles are contiguous in tile order (octant order under ConstRho)
+  std::vector<int> chunk_begin;
+  std::vector<int4> chunk;
+  const std::vector<unsigned int> zero(nmembers, 0u);
   {
     const int l = max_level;
     const int tpb = padded ? ((NP + kTile - 1) / kTile) * ((NP + kTile - 1) / kTile) * ((NP + kTile - 1) / kTile) : 1;
@@ -1099,19 +1103,21 @@ void octlb_dev::Prepare() {
     }
     if (!padded)
       for (int& t : tiles_of) t *= kTile;  // a partial per x plane
-    std::vector<int> chunk_begin;
-    const std::vector<int4> chunk = StatChunks(fast_stats ? tiles_of : cells, &chunk_begin);
-    stat_chunks = static_cast<int>(chunk.size());
-    d_stat_chunk = PAlloc<int4>(chunk.size());
-    Upload(d_stat_chunk, chunk, stream);
-    d_stat_chunk_begin = PAlloc<int>(chunk_begin.size());
-    Upload(d_stat_chunk_begin, chunk_begin, stream);
-    d_stat_part = PAlloc<StatPart>(chunk.size());
-    d_stat_sum = PAlloc<double2>(chunk.size());
-    const std::vector<unsigned int> zero(nmembers, 0u);
-    d_stat_done = PAlloc<unsigned int>(zero.size());
-    Upload(d_stat_done, zero, stream);
-    Sync();  // the tables above leave scope
+    if (sc.const_rho) {
+      chunk = StatChunks(fast_stats ? tiles_of : cells, &chunk_begin);
+      stat_chunks = static_cast<int>(chunk.size());
+      d_stat_chunk = PAlloc<int4>(chunk.size());
+      Upload(d_stat_chunk, chunk, stream);
+      d_stat_chunk_begin = PAlloc<int>(chunk_begin.size());
+      Upload(d_stat_chunk_begin, chunk_begin, stream);
+      if (fast_stats) {
+        d_stat_sum = PAlloc<double2>(chunk.size());
+        d_stat_done = PAlloc<unsigned int>(zero.size());
+        Upload(d_stat_done, zero, stream);
+      } else {
+        d_stat_part = PAlloc<StatPart>(chunk.size());
+      }
+    }
   }
   Upload(d_bt, bt, stream);
   Sync();
