@@ -14,6 +14,7 @@
 // whole 10^3 box and writes S of step n to the other buffer.
 #include "lbm_device.h"
 #include "adjoint_ml.h"
+#include "launch.h"
 
 #include <algorithm>
 
@@ -1001,7 +1002,7 @@ constexpr int kFdThreads = 256;
 template <typename T>
 __global__ __launch_bounds__(kFdThreads) void KFd(FdArgs<T> a, int begin, int count) {
   BumpStep(a.step, a.step_next);
-  const int g = static_cast<int>(blockIdx.x * kFdThreads + threadIdx.x) / kFdLanes;
+  const int g = static_cast<int>(blockIdx.x * (kFdThreads / kFdLanes) + threadIdx.x / kFdLanes);
   const int lane = threadIdx.x % kFdLanes;
   const bool live = g < count;  // the last groups repeat a cell: every lane takes part in the shuffles
   const int e = begin + (live ? g : count - 1);
@@ -1971,8 +1972,14 @@ template <typename T>
 void LaunchFd(const FdArgs<T>& a, const int* phase_begin, hipStream_t s) {
   for (int ph = 0; ph < 3; ++ph) {
     const int cnt = phase_begin[ph + 1] - phase_begin[ph];
-    if (cnt > 0) hipLaunchKernelGGL(KFd<T>, Grid(static_cast<long long>(cnt) * kFdLanes, kFdThreads), dim3(kFdThreads), 0, s, a,
-                         phase_begin[ph], cnt);
+    // 16 lanes a cell: one launch holds 268 million cells
+    constexpr int kCells = kFdThreads / kFdLanes;
+    ForLaunches((static_cast<int64_t>(cnt) + kCells - 1) / kCells, kFdThreads, [&](int64_t first, int64_t groups) {
+      const int64_t at = first * kCells;
+      hipLaunchKernelGGL(KFd<T>, dim3(static_cast<unsigned>(groups)), dim3(kFdThreads), 0, s, a,
+                         static_cast<int>(phase_begin[ph] + at),
+                         static_cast<int>(std::min<int64_t>(cnt - at, groups * kCells)));
+    });
   }
   const int total = phase_begin[3];
   if (total > 0) hipLaunchKernelGGL(KFdCommit<T>, Grid(total, 256), dim3(256), 0, s, a, total);
@@ -2029,11 +2036,12 @@ void LaunchMass(const T* p0, const T* p1, const ParArray& par, const BlockTab* b
 constexpr int kMacroPad = 73;  // LDS doubles per x plane: the transposed reads spread over the banks
 template <typename T>
 __global__ __launch_bounds__(kTileCells) void KMacro(const T* pops0, const T* pops1, ParArray par,
-                                                     const BlockTab* bt, SimConst sc, int tpe, double* rho,
-                                                     double* u) {
+                                                     const BlockTab* bt, SimConst sc, int tpe, unsigned int first,
+                                                     double* rho, double* u) {
   __shared__ double lds[4][kTile * kMacroPad];
   const int tpb = tpe * tpe * tpe;
-  const int b = blockIdx.x / tpb, w = blockIdx.x % tpb, n = sc.n;
+  const unsigned int tile = first + blockIdx.x;
+  const int b = static_cast<int>(tile / tpb), w = static_cast<int>(tile % tpb), n = sc.n;
   const int x0 = w / (tpe * tpe) * kTile, y0 = (w / tpe) % tpe * kTile, z0 = w % tpe * kTile;
   const T* base = (par.v[bt[b].level] ? pops1 : pops0) + static_cast<size_t>(b) * kQ * sc.plane;
   const int tid = threadIdx.x;
@@ -2070,8 +2078,10 @@ template <typename T>
 void LaunchMacro(const T* p0, const T* p1, const ParArray& par, const BlockTab* bt, const SimConst& sc, int nb,
                  double* rho, double* u, hipStream_t s) {
   const int tpe = (sc.n + kTile - 1) / kTile;
-  hipLaunchKernelGGL(KMacro<T>, dim3(static_cast<unsigned>(nb) * tpe * tpe * tpe), dim3(kTileCells), 0, s, p0, p1, par,
-                     bt, sc, tpe, rho, u);
+  ForLaunches(static_cast<int64_t>(nb) * tpe * tpe * tpe, kTileCells, [&](int64_t first, int64_t tiles) {
+    hipLaunchKernelGGL(KMacro<T>, dim3(static_cast<unsigned>(tiles)), dim3(kTileCells), 0, s, p0, p1, par, bt, sc, tpe,
+                       static_cast<unsigned>(first), rho, u);
+  });
 }
 
 #define OCTLB_INSTANTIATE(T)                                                                      \
