@@ -1424,10 +1424,8 @@ struct octlb_adj {
     return a;
   }
 
-  // operation k forward on (x, y, prev) at time t; when tape is given (in
-  // state coordinates: entry e of the window at tape[e]), the window of the
-  // state that the operation's adjoint reads is copied there first, and for a
-  // prolongation the prev macros into ptape
+  // Bouzidi rows [k0, k1) behind y's entries, multiply read entries' lists [o0,
+  // o1) behind d_lx's
   template <typename S>
   void LinkRows(S* y, int k0, int k1) {
     if (k1 > k0)
@@ -1438,6 +1436,11 @@ struct octlb_adj {
       hipLaunchKernelGGL(KAdjReaders, dim3(Blocks(o1 - o0)), dim3(kThreads), 0, stream, d_lx, d_ovo, d_ove, d_links, o0,
                          o1, ntot);
   }
+
+  // operation k forward on (x, y, prev) at time t; when tape is given (in
+  // state coordinates: entry e of the window at tape[e]), the window of the
+  // state that the operation's adjoint reads is copied there first, and for a
+  // prolongation the prev macros into ptape
   template <typename S>
   void MLApply(size_t k, S* x, S* y, S* prev, double t, S* tape, S* ptape) {
     const size_t pm = static_cast<size_t>(npts) * kMacro;

@@ -1129,13 +1129,6 @@ struct FdLds {
     const int c = (Mirror(x, n) * n + Mirror(y, n)) * n + Mirror(z, n);
     return (slot[c] >= 0 && c < self) ? rho_post[c] : rho_pre[c];
   }
-  __device__ void ComputeRhoU(int x, int y, int z, T& rho, T* u) const {
-    const int c = (x * kTile + y) * kTile + z;
-    rho = ComputeRho(x, y, z);
-    u[0] = ux[c];
-    u[1] = uy[c];
-    u[2] = uz[c];
-  }
   __device__ void NormalGrad(int x, int y, int z, int axis, int normal, T* g) const {
     const int ox = axis == 0 ? -normal : 0, oy = axis == 1 ? -normal : 0, oz = axis == 2 ? -normal : 0;
     T u0[3], u1[3], u2[3];
