@@ -363,10 +363,6 @@ def cpu_baseline(case, budget_s):
                               "sample": f"{s1} coarse steps, 1 thread, {dt1:.1f} s"}}
 
 
-FP64_VALU_PEAK_GFLOPS = 78600.0
-FLOPS_PER_CELL_TRIANGLE = 101  # 3 edges x (closest point 23 + distance 8) + distance 8
-
-
 def run_migrate(precision=32, mark_frac=0.1, seed=3, reps=3):
     """State migration after a forest change (octlb_dev_migrate) on the
     synthetic 3-level forest: a seeded 10% of its level-1 blocks refined
@@ -462,7 +458,6 @@ def run_link_build(with_cpu, segments=512, rings=8, reps=3, cpu_blocks=24):
         ex, ey, ez = cases.C[i]
         near |= pad[:, 1 + ez:9 + ez, 1 + ey:9 + ey, 1 + ex:9 + ex]
     ncand = int((near & ~solid).sum())
-    gflops = ncand * tris.shape[0] * FLOPS_PER_CELL_TRIANGLE / gpu_s / 1e9
     out = {
         "workload": ("cylinder-channel forest (1,152 blocks of 8^3), z-spanning cylinder D=16 fine cells "
                      f"as {tris.shape[0]} triangles ({segments} segments x {rings} rings); material voxelized "
@@ -472,9 +467,6 @@ def run_link_build(with_cpu, segments=512, rings=8, reps=3, cpu_blocks=24):
         "links": int(len(link)),
         "gpu_ms": round(gpu_s * 1e3, 3),
         "voxelize": vox,
-        "roofline": {"bound": "fp64 valu", "achieved": round(gflops, 1), "peak": FP64_VALU_PEAK_GFLOPS,
-                     "unit": "GFLOP/s", "frac": round(gflops / FP64_VALU_PEAK_GFLOPS, 4),
-                     "flops_per_cell_triangle": FLOPS_PER_CELL_TRIANGLE},
     }
     if with_cpu:
         from oracle.binding import build_links as oracle_links
