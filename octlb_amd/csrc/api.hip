@@ -195,7 +195,6 @@ struct octlb_dev {
   int* d_stat_chunk_begin = nullptr;  // [nmembers + 1]
   StatPart* d_stat_part = nullptr;
   double2* d_stat_sum = nullptr;
-  unsigned int* d_stat_done = nullptr;  // [nmembers]
   int stat_chunks = 0;
   int* d_step = nullptr;   // [2]: double-buffered coarse-step counter
   int step_slot = 0;       // slot holding the current step's time
@@ -1071,7 +1070,6 @@ void octlb_dev::Prepare() {
   // tiles are contiguous in tile order (octant order under ConstRho)
   std::vector<int> chunk_begin;
   std::vector<int4> chunk;
-  const std::vector<unsigned int> zero(nmembers, 0u);
   {
     const int l = max_level;
     const int tpb = padded ? ((NP + kTile - 1) / kTile) * ((NP + kTile - 1) / kTile) * ((NP + kTile - 1) / kTile) : 1;
@@ -1104,7 +1102,7 @@ void octlb_dev::Prepare() {
     if (!padded)
       for (int& t : tiles_of) t *= kTile;  // a partial per x plane
     if (sc.const_rho) {
-      chunk = StatChunks(fast_stats ? tiles_of : cells, &chunk_begin);
+      chunk = StatChunks(fast_stats ? tiles_of : cells, fast_stats, &chunk_begin);
       stat_chunks = static_cast<int>(chunk.size());
       d_stat_chunk = PAlloc<int4>(chunk.size());
       Upload(d_stat_chunk, chunk, stream);
@@ -1112,8 +1110,6 @@ void octlb_dev::Prepare() {
       Upload(d_stat_chunk_begin, chunk_begin, stream);
       if (fast_stats) {
         d_stat_sum = PAlloc<double2>(chunk.size());
-        d_stat_done = PAlloc<unsigned int>(zero.size());
-        Upload(d_stat_done, zero, stream);
       } else {
         d_stat_part = PAlloc<StatPart>(chunk.size());
       }
@@ -1384,8 +1380,7 @@ void octlb_dev::Level(int l) {
     }
     par[l] ^= 1;
     if (a.want_stats == 1)
-      LaunchStatsFinalize(d_stats, d_stat_chunk, d_stat_chunk_begin, stat_chunks, d_stat_sum, d_stat_done, d_avg,
-                          stream);
+      LaunchStatsFinalize(d_stats, d_stat_chunk, d_stat_chunk_begin, stat_chunks, nmembers, d_stat_sum, d_avg, stream);
     if (a.want_stats == 2)
       LaunchStatsSequential(d_stat_val, d_stat_use, d_stat_chunk, d_stat_chunk_begin, stat_chunks, nmembers,
                             d_stat_part, d_avg, stream);

@@ -591,7 +591,9 @@ __global__ __launch_bounds__(512) void KPadded(TileArgs<T> a) {
 }
 
 // ------------------------------------------------------------ small kernels
-constexpr int kStatChunk = 1024;  // cells (ordered sum) or partials (fast) per chunk
+constexpr int kStatChunk = 1024;   // cells per chunk of the ordered sum
+constexpr int kFastChunk = 4096;   // partials per chunk of the fast one
+constexpr int kFastThreads = 1024;
 constexpr int kStatChunkThreads = 256;
 
 // Sum of a workgroup's (s, c) in a fixed order, in thread 0.
@@ -607,55 +609,58 @@ __device__ inline void GroupSum(double& s, double& c, double* rs, double* rc) {
   }
   __syncthreads();
   if (threadIdx.x == 0)
-    for (int k = 1; k < kStatChunkThreads / 64; ++k) {
+    for (int k = 1; k < kFastThreads / 64; ++k) {
       s += rs[k];
       c += rc[k];
     }
-  __syncthreads();  // rs, rc may be written again
 }
 
 // Tree reduction of the partial sums (fast_stats: not the reference's
 // summation order, but a fixed one): a workgroup per chunk of a member's
-// partials, the last of a member to finish (a device-scope counter, reset by it)
-// sums the chunks.  There is a partial for every 64 cells, and one workgroup
-// per member was bound by its own loads: a step of 224^3 cells took 927 us that
-// way and takes 647 us (FP32).
-__global__ __launch_bounds__(kStatChunkThreads) void KStatsFinalize(const double2* partial, const int4* chunk,
-                                                                    const int* chunk_begin, double2* sums,
-                                                                    unsigned int* done, double* avg) {
-  __shared__ double rs[kStatChunkThreads / 64], rc[kStatChunkThreads / 64];
-  __shared__ int last;
+// partials, then one per member if any has several chunks (more than 64^3 cells).
+// There is a partial for every 64 cells, and 256 threads per member were bound by
+// their own loads: a step of 224^3 cells took 927 us that way and takes 640 us
+// (FP32).  Letting the last workgroup of a member sum its chunks costs a
+// device-scope fence in every workgroup: 24 us for 64 members of up to 96^3 cells,
+// where the two launches take 11 us (5.3 us, one launch, for 12 of up to 64^3).
+__device__ inline double StatAverage(double s, double c) {
+  return c > 0.0 ? s / c : 1.0;  // CollideRhoStats::average (block_lattice.h:31)
+}
+
+__global__ __launch_bounds__(kFastThreads) void KStatsSums(const double2* partial, const int4* chunk,
+                                                                const int* chunk_begin, double2* sums, double* avg) {
+  __shared__ double rs[kFastThreads / 64], rc[kFastThreads / 64];
   const int4 ch = chunk[blockIdx.x];  // first partial, end, member
-  const int m = ch.z, tid = threadIdx.x;
-  const int cb = chunk_begin[m], nc = chunk_begin[m + 1] - cb;
   double s = 0.0, c = 0.0;
 #pragma unroll
-  for (int k = 0; k < kStatChunk / kStatChunkThreads; ++k) {
-    const int i = ch.x + k * kStatChunkThreads + tid;
+  for (int k = 0; k < kFastChunk / kFastThreads; ++k) {
+    const int i = ch.x + k * kFastThreads + static_cast<int>(threadIdx.x);
     if (i < ch.y) {
       s += partial[i].x;
       c += partial[i].y;
     }
   }
   GroupSum(s, c, rs, rc);
-  if (nc > 1) {
-    if (tid == 0) {
-      sums[blockIdx.x] = make_double2(s, c);
-      __threadfence();  // the chunk's sum before the count that publishes it
-      last = atomicAdd(&done[m], 1u) == static_cast<unsigned int>(nc - 1);
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();  // every chunk's sum is visible to the last workgroup
-    s = c = 0.0;
-    for (int k = tid; k < nc; k += kStatChunkThreads) {
-      s += sums[cb + k].x;
-      c += sums[cb + k].y;
-    }
-    GroupSum(s, c, rs, rc);
-    if (tid == 0) done[m] = 0u;
+  if (threadIdx.x != 0) return;
+  if (chunk_begin[ch.z + 1] - chunk_begin[ch.z] > 1) {
+    sums[blockIdx.x] = make_double2(s, c);
+  } else {
+    avg[ch.z] = StatAverage(s, c);
   }
-  if (tid == 0) avg[m] = c > 0.0 ? s / c : 1.0;  // CollideRhoStats::average (block_lattice.h:31)
+}
+
+__global__ __launch_bounds__(kFastThreads) void KStatsFinalize(const int* chunk_begin, const double2* sums,
+                                                                    double* avg) {
+  __shared__ double rs[kFastThreads / 64], rc[kFastThreads / 64];
+  const int m = blockIdx.x, cb = chunk_begin[m], ce = chunk_begin[m + 1];
+  if (ce - cb <= 1) return;
+  double s = 0.0, c = 0.0;
+  for (int k = cb + static_cast<int>(threadIdx.x); k < ce; k += kFastThreads) {
+    s += sums[k].x;
+    c += sums[k].y;
+  }
+  GroupSum(s, c, rs, rc);
+  if (threadIdx.x == 0) avg[m] = StatAverage(s, c);
 }
 
 // CollideRhoStats accumulated in the reference's cell order (blocks of the
@@ -1902,18 +1907,21 @@ void LaunchTile(const TileArgs<T>& a, hipStream_t s) {
 
 static inline dim3 Grid(long long n, int bs) { return dim3(static_cast<unsigned>((n + bs - 1) / bs)); }
 
-void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, double2* sums,
-                         unsigned int* done, double* avg, hipStream_t s) {
-  hipLaunchKernelGGL(KStatsFinalize, dim3(nchunk), dim3(kStatChunkThreads), 0, s,
-                     reinterpret_cast<const double2*>(partial), chunk, chunk_begin, sums, done, avg);
+void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, int members,
+                         double2* sums, double* avg, hipStream_t s) {
+  hipLaunchKernelGGL(KStatsSums, dim3(nchunk), dim3(kFastThreads), 0, s,
+                     reinterpret_cast<const double2*>(partial), chunk, chunk_begin, sums, avg);
+  if (nchunk > members)
+    hipLaunchKernelGGL(KStatsFinalize, dim3(members), dim3(kFastThreads), 0, s, chunk_begin, sums, avg);
 }
 
-std::vector<int4> StatChunks(const std::vector<int>& begin, std::vector<int>* chunk_begin) {
+std::vector<int4> StatChunks(const std::vector<int>& begin, bool fast, std::vector<int>* chunk_begin) {
+  const int per = fast ? kFastChunk : kStatChunk;
   std::vector<int4> chunk;
   chunk_begin->assign(1, 0);
   for (size_t m = 0; m + 1 < begin.size(); ++m) {
-    for (int k = begin[m]; k < begin[m + 1]; k += kStatChunk)
-      chunk.push_back(make_int4(k, std::min(k + kStatChunk, begin[m + 1]), static_cast<int>(m), k - begin[m]));
+    for (int k = begin[m]; k < begin[m + 1]; k += per)
+      chunk.push_back(make_int4(k, std::min(k + per, begin[m + 1]), static_cast<int>(m), k - begin[m]));
     chunk_begin->push_back(static_cast<int>(chunk.size()));
   }
   return chunk;

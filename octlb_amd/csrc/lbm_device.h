@@ -490,10 +490,9 @@ void LaunchTile(const TileArgs<T>& a, hipStream_t s);
 // ConstRho averages of the members.  Both sums go by chunks of a member's
 // partials (fast) or cells (reference order): (first, end, member, how many of
 // the member's before it), member m owning begin[m] .. begin[m + 1] and chunks
-// [chunk_begin[m], chunk_begin[m + 1]); sums and part hold one entry per chunk,
-// done one zero per member.
-void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, double2* sums,
-                         unsigned int* done, double* avg, hipStream_t s);
+// [chunk_begin[m], chunk_begin[m + 1]); sums and part hold one entry per chunk.
+void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, int members,
+                         double2* sums, double* avg, hipStream_t s);
 struct StatPair {
   long long d0, d1;  // what the chunk adds to an even / odd integer sum
 };
@@ -502,7 +501,7 @@ struct StatPart {
   int count;
   int e;  // exponent of the running sum the pair holds for
 };
-std::vector<int4> StatChunks(const std::vector<int>& begin, std::vector<int>* chunk_begin);
+std::vector<int4> StatChunks(const std::vector<int>& begin, bool fast, std::vector<int>* chunk_begin);
 void LaunchStatsSequential(const double* val, const uint8_t* use, const int4* chunk, const int* chunk_begin,
                            int nchunk, int members, StatPart* part, double* avg, hipStream_t s);
 void LaunchStepInc(const int* step, int* step_next, hipStream_t s);

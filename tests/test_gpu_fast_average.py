@@ -1,6 +1,5 @@
-"""The ConstRho average summed by chunks of 1,024 partials (fast_stats), a
-partial per x plane of a block: members of less than a chunk, just below and
-above one, several; step by step and from a captured graph, against the average
+"""The ConstRho average summed by chunks of 4,096 partials (fast_stats), a
+partial per x plane of a block: members of less than a chunk, exactly one, several; step by step and from a captured graph, against the average
 in the reference's order.  N positive values summed in any order are within
 (N - 1) 2^-53 of the exact sum, so the two differ by at most twice that, once per
 step taken."""
@@ -22,8 +21,8 @@ def _solver(sizes, precision, fast):
     return s
 
 
-# 8 partials, 1,000 and 1,728 (a chunk is 1,024), 4 chunks; members of both kinds
-@pytest.mark.parametrize("sizes", [(8,), (40,), (48,), (64,), (48, 8, 40, 56)])
+# 8 partials, 1,000, 4,096 (a whole chunk), 5,832 (two chunks), 13,824; members of both kinds
+@pytest.mark.parametrize("sizes", [(8,), (40,), (64,), (72,), (96,), (48, 8, 72, 40)])
 @pytest.mark.parametrize("precision", [64, 32])
 def test_matches_the_ordered_average(sizes, precision):
     fast, ordered = _solver(sizes, precision, 1), _solver(sizes, precision, 0)
