@@ -246,7 +246,8 @@ struct VoxArgs {
   int channel;          // internal channel (else external obstacle)
   uint8_t* material;
   int* queue;           // cells the filters left open: index into material
-  unsigned int* queued;
+  unsigned int room;    // how many the queue holds
+  unsigned int* queued; // how many there are
 };
 
 // Lists a box [lo, hi] (of a triangle or of a group) belongs to for the tile
@@ -418,7 +419,8 @@ __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
     if (m >= 0) {
       a.material[material_at(c)] = static_cast<uint8_t>(m);
     } else {
-      a.queue[atomicAdd(a.queued, 1u)] = static_cast<int>(material_at(c));
+      const unsigned int slot = atomicAdd(a.queued, 1u);
+      if (slot < a.room) a.queue[slot] = static_cast<int>(material_at(c));
     }
   }
 }
@@ -523,27 +525,31 @@ __global__ void KSampleInside(const VTri* tris, int64_t nouter, const double* bo
   inside[q] = votes >= 2 ? 1 : 0;
 }
 
-// Device memory of one call, one allocation carved into 256-byte aligned arrays.
+// Device memory of one call, an allocation per array.  One for all of them is
+// beyond the 2 MB that the runtime hands out of blocks it keeps: freed by every
+// call, it left the copies of pageable memory slow, here and in the calls that
+// follow (290 KB: 118 instead of 17 us; voxelizer and link build of 1,152 blocks
+// 2.1 ms that way, 1.0 ms this way).
 class VoxBuffer {
  public:
-  size_t Add(size_t bytes) {
-    const size_t at = size_;
-    size_ += (bytes + 255) & ~static_cast<size_t>(255);
-    return at;
-  }
-  void Alloc() { VOX_CHECK(hipMalloc(&base_, size_)); }
   template <typename P>
-  P* At(size_t offset) const {
-    return reinterpret_cast<P*>(static_cast<char*>(base_) + offset);
+  P* Get(size_t count) {
+    void* p = nullptr;
+    VOX_CHECK(hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(P)));
+    ptrs_.push_back(p);
+    return static_cast<P*>(p);
   }
   ~VoxBuffer() {
-    if (base_) (void)hipFree(base_);
+    for (void* p : ptrs_) (void)hipFree(p);  // teardown
   }
 
  private:
-  void* base_ = nullptr;
-  size_t size_ = 0;
+  std::vector<void*> ptrs_;
 };
+
+// Open cells that a call keeps room for; where there are more, the filters run
+// again with room for all.
+constexpr size_t kOpenRoom = 131072;
 
 constexpr double kMinLumenOutsideFraction = 0.05;  // part_voxelizer.cpp:10-11
 constexpr int kWatertightSampleResolution = 5;
@@ -570,29 +576,18 @@ int VoxelizePart(int32_t num_blocks, int32_t n, const double* bounds, int64_t nu
   const int te = (n + kVoxTile - 1) / kVoxTile;
   const int64_t ntile = static_cast<int64_t>(num_blocks) * te * te * te;
   const int64_t ngroup = (ntri + kGroup - 1) / kGroup;
-  const int pts = kWatertightSampleResolution * kWatertightSampleResolution * kWatertightSampleResolution;
   VoxBuffer buf;
-  const size_t o_raw = buf.Add(static_cast<size_t>(ntri) * 9 * sizeof(double));
-  const size_t o_tri = buf.Add(static_cast<size_t>(ntri) * sizeof(VTri));
-  const size_t o_box = buf.Add(static_cast<size_t>(ntri) * 6 * sizeof(double));
-  const size_t o_gbox = buf.Add(static_cast<size_t>(ngroup) * 6 * sizeof(double));
-  const size_t o_bounds = buf.Add(static_cast<size_t>(num_blocks) * 6 * sizeof(double));
-  const size_t o_mat = buf.Add(total);
-  const size_t o_queue = buf.Add(total * sizeof(int));
-  const size_t o_queued = buf.Add(sizeof(unsigned int));
-  const size_t o_sbox = buf.Add(6 * sizeof(double));
-  const size_t o_in = buf.Add(static_cast<size_t>(pts) * sizeof(int));
-  buf.Alloc();
-  double* d_raw = buf.At<double>(o_raw);
+  double* d_raw = buf.Get<double>(static_cast<size_t>(ntri) * 9);
   VOX_CHECK(hipMemcpy(d_raw, triangles, static_cast<size_t>(num_triangles) * 9 * sizeof(double),
                       hipMemcpyHostToDevice));
   if (num_inner > 0)
     VOX_CHECK(hipMemcpy(d_raw + num_triangles * 9, inner, static_cast<size_t>(num_inner) * 9 * sizeof(double),
                         hipMemcpyHostToDevice));
-  VTri* d_tri = buf.At<VTri>(o_tri);
+  VTri* d_tri = buf.Get<VTri>(static_cast<size_t>(ntri));
+  double* d_tribox = buf.Get<double>(static_cast<size_t>(ntri) * 6);
+  double* d_gbox = buf.Get<double>(static_cast<size_t>(ngroup) * 6);
   hipLaunchKernelGGL(KTriPrep, dim3(static_cast<unsigned>((ntri + kVoxThreads - 1) / kVoxThreads)), dim3(kVoxThreads),
-                     0, nullptr, d_raw, ntri, num_triangles, d_tri, buf.At<double>(o_box), buf.At<double>(o_gbox),
-                     ngroup);
+                     0, nullptr, d_raw, ntri, num_triangles, d_tri, d_tribox, d_gbox, ngroup);
   VOX_CHECK(hipGetLastError());
 
   if (channel) {
@@ -604,8 +599,9 @@ int VoxelizePart(int32_t num_blocks, int32_t n, const double* bounds, int64_t nu
         box[3 + d] = std::max(box[3 + d], triangles[t * 3 + d]);
       }
     const int s = kWatertightSampleResolution;
-    double* d_box = buf.At<double>(o_sbox);
-    int* d_in = buf.At<int>(o_in);
+    const int pts = s * s * s;
+    double* d_box = buf.Get<double>(6);
+    int* d_in = buf.Get<int>(pts);
     VOX_CHECK(hipMemcpy(d_box, box, sizeof(box), hipMemcpyHostToDevice));
     hipLaunchKernelGGL(KSampleInside, dim3((pts + 63) / 64), dim3(64), 0, nullptr, d_tri, num_triangles, d_box, s,
                        d_in);
@@ -621,20 +617,21 @@ int VoxelizePart(int32_t num_blocks, int32_t n, const double* bounds, int64_t nu
 
   VoxArgs a{};
   a.tris = d_tri;
-  a.box = buf.At<double>(o_box);
-  a.gbox = buf.At<double>(o_gbox);
+  a.box = d_tribox;
+  a.gbox = d_gbox;
   a.ntri = ntri;
   a.ngroup = static_cast<int>(ngroup);
-  a.bounds = buf.At<double>(o_bounds);
+  double* d_bounds = buf.Get<double>(static_cast<size_t>(num_blocks) * 6);
+  a.bounds = d_bounds;
   a.n = n;
   a.te = te;
   a.channel = channel ? 1 : 0;
-  a.material = buf.At<uint8_t>(o_mat);
-  a.queue = buf.At<int>(o_queue);
-  a.queued = buf.At<unsigned int>(o_queued);
-  VOX_CHECK(hipMemcpy(buf.At<double>(o_bounds), bounds, static_cast<size_t>(num_blocks) * 6 * sizeof(double),
+  a.material = buf.Get<uint8_t>(total);
+  a.room = static_cast<unsigned int>(std::min(total, kOpenRoom));
+  a.queue = buf.Get<int>(a.room);
+  a.queued = buf.Get<unsigned int>(1);
+  VOX_CHECK(hipMemcpy(d_bounds, bounds, static_cast<size_t>(num_blocks) * 6 * sizeof(double),
                       hipMemcpyHostToDevice));
-  VOX_CHECK(hipMemset(a.queued, 0, sizeof(unsigned int)));
   // blocks of 9^3 or 10^3 cells have eight tiles, most of their cells idle:
   // 1.6e9 cells are 17.6 million workgroups
   auto launch = [&](auto kernel, int64_t groups, int threads) {
@@ -644,9 +641,18 @@ int VoxelizePart(int32_t num_blocks, int32_t n, const double* bounds, int64_t nu
       VOX_CHECK(hipGetLastError());
     });
   };
-  launch(KClassify, ntile, kVoxThreads);
   unsigned int queued = 0;
-  VOX_CHECK(hipMemcpy(&queued, a.queued, sizeof(queued), hipMemcpyDeviceToHost));
+  auto classify = [&] {
+    VOX_CHECK(hipMemset(a.queued, 0, sizeof(unsigned int)));
+    launch(KClassify, ntile, kVoxThreads);
+    VOX_CHECK(hipMemcpy(&queued, a.queued, sizeof(queued), hipMemcpyDeviceToHost));
+  };
+  classify();
+  if (queued > a.room) {
+    a.room = queued;
+    a.queue = buf.Get<int>(queued);
+    classify();
+  }
   launch(KClassifyExact, queued, 64);
   VOX_CHECK(hipMemcpy(material, a.material, total, hipMemcpyDeviceToHost));
   if (num_exact) *num_exact = queued;

@@ -45,3 +45,17 @@ def test_channel(n):
     np.testing.assert_array_equal(got, binding.voxelize_part(*args))
     if n != 9:
         assert exact > 0
+
+
+def test_more_open_cells_than_the_first_room():
+    """More cells than the call's first queue holds (131,072), against the same
+    blocks in calls that each stay below."""
+    k = 46
+    at = np.stack(np.meshgrid(*[np.arange(k)] * 3, indexing="ij"), -1).reshape(-1, 3) / k
+    bounds = np.concatenate([at, at + 1.0 / k], 1)
+    soup = geometry.sphere_soup(CENTRE, 0.375, 4)
+    got, exact = geometry.voxelize_part(bounds, 8, soup, geometry.PART_EXTERNAL_OBSTACLE)
+    parts = [geometry.voxelize_part(b, 8, soup, geometry.PART_EXTERNAL_OBSTACLE) for b in np.array_split(bounds, 24)]
+    assert exact > 131072 > max(n for _, n in parts)
+    assert exact == sum(n for _, n in parts)
+    assert np.array_equal(got, np.concatenate([m for m, _ in parts]))
