@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kVoxThreads) void KTriPrep(const double* tri, int64
 // ------------------------------------------------------------ classification
 constexpr int kVoxTile = 8;
 constexpr int kVoxCells = kVoxTile * kVoxTile * kVoxTile;
-constexpr int kVoxLanes = 8;      // lanes per candidate triangle
+constexpr int kVoxLanes = 3;      // log2 of the fewest lanes per candidate triangle
 constexpr int kVoxQueue = 2048;   // candidates staged in LDS; one round of the waves adds at most 1,024
 
 // state bits of a cell
@@ -240,6 +240,7 @@ struct VoxArgs {
   int64_t ntri;
   int ngroup;
   const double* bounds;
+  int nb;
   int n;
   int te;               // tiles per block edge
   int first;            // the launch's first tile (queue entry)
@@ -285,9 +286,11 @@ __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
   __shared__ int groups[kVoxThreads];
   __shared__ int nq, ng;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n = a.n, tpb = a.te * a.te * a.te;
+  const int n = a.n;
   const int tile = a.first + static_cast<int>(blockIdx.x);
-  const int b = tile / tpb, tt = tile % tpb;
+  // the same tile of all blocks, then the next: with a block's tiles side by
+  // side, those of the same size would all fall to one XCD
+  const int b = tile % a.nb, tt = tile / a.nb;
   // tiles in MaterialField order: x fastest
   const int org[3] = {tt % a.te * kVoxTile, tt / a.te % a.te * kVoxTile, tt / (a.te * a.te) * kVoxTile};
   int ext[3];
@@ -313,8 +316,14 @@ __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
   __syncthreads();
   const double tb[6] = {cl[0][0], cl[1][0], cl[2][0], ch[0][ext[0] - 1], ch[1][ext[1] - 1], ch[2][ext[2] - 1]};
 
+  // The lanes of a candidate, 8 to 64, go over the cells in its reach: as many as
+  // leave none idle where few candidates with long reaches (the faces of a box)
+  // meet the tile.
   auto work = [&](int count) {
-    for (int q = tid / kVoxLanes; q < count; q += kVoxThreads / kVoxLanes) {
+    int ls = kVoxLanes;  // log2 of them
+    while (ls < 6 && (count << ls) * 2 <= kVoxThreads) ++ls;
+    const int lanes = 1 << ls, w0 = tid & (lanes - 1);
+    for (int q = tid >> ls; q < count; q += kVoxThreads >> ls) {
       const VTri& t = a.tris[VoxTriangle(queue[q])];
       const int l = VoxList(queue[q]);
       int lo[3], hi[3];  // the cells in reach, per axis
@@ -336,8 +345,23 @@ __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
       }
       const int ni = hi[0] - lo[0], nj = hi[1] - lo[1], nk = hi[2] - lo[2];
       if (ni <= 0 || nj <= 0 || nk <= 0) continue;
-      for (int w = tid % kVoxLanes; w < ni * nj * nk; w += kVoxLanes) {
-        const int i = lo[0] + w % ni, j = lo[1] + w / ni % nj, k = lo[2] + w / (ni * nj);
+      // cells w0, w0 + lanes, ... of the reach, x fastest: stepped with carries
+      const int si = lanes % ni, sj = lanes / ni % nj, sk = lanes / (ni * nj);
+      int ri = w0 % ni - si, rj = w0 / ni % nj - sj, rk = w0 / (ni * nj) - sk;
+      for (;;) {
+        ri += si;
+        rj += sj;
+        rk += sk;
+        if (ri >= ni) {
+          ri -= ni;
+          ++rj;
+        }
+        if (rj >= nj) {
+          rj -= nj;
+          ++rk;
+        }
+        if (rk >= nk) break;
+        const int i = lo[0] + ri, j = lo[1] + rj, k = lo[2] + rk;
         const int c = (k * kVoxTile + j) * kVoxTile + i;
         if (st[c] & kBitHit) continue;  // a boundary cell already
         if (l == 0) {
@@ -623,6 +647,7 @@ int VoxelizePart(int32_t num_blocks, int32_t n, const double* bounds, int64_t nu
   a.ngroup = static_cast<int>(ngroup);
   double* d_bounds = buf.Get<double>(static_cast<size_t>(num_blocks) * 6);
   a.bounds = d_bounds;
+  a.nb = num_blocks;
   a.n = n;
   a.te = te;
   a.channel = channel ? 1 : 0;
