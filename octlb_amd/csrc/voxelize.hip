@@ -26,7 +26,8 @@
 // box per 64 triangles; (2) one workgroup per 8^3 tile of cells picks the
 // triangles that can matter to the tile (group boxes, then triangle boxes)
 // and, triangle by triangle, tests the few cells each one can reach,
-// collecting hits, parities and undecided filters as bits per cell; (3) one
+// collecting hits, parities and undecided filters as bits per cell (few
+// triangles and many blocks: a thread per cell instead); (3) one
 // wave per cell whose filters could not decide repeats its classification with
 // exact fallbacks, its lanes a candidate triangle each.
 //
@@ -233,6 +234,24 @@ constexpr uint32_t kBitHit = 1u, kBitOpen = 2u;
 __device__ inline uint32_t OddBit(int mesh, int ax) { return 4u << (mesh * 3 + ax); }
 __device__ inline uint32_t UnsureBit(int mesh, int ax) { return 256u << (mesh * 3 + ax); }
 
+// The material of a cell with these bits, or -1 if the filters left it open.
+__device__ inline int Decide(uint32_t s, int channel) {
+  if (s & kBitHit) return kBoundary;
+  if (s & kBitOpen) return -1;
+  // inside votes: decided when the certain axes settle the majority
+  int inside[2];
+  for (int q = 0; q < 2; ++q) {
+    int yes = 0, no = 0;
+    for (int ax = 0; ax < 3; ++ax) {
+      if (s & UnsureBit(q, ax)) continue;
+      if (s & OddBit(q, ax)) ++yes; else ++no;
+    }
+    inside[q] = yes >= 2 ? 1 : (no >= 2 ? 0 : -1);
+  }
+  if (channel && inside[1] != 0) return inside[1] < 0 ? -1 : kFluid;  // lumen
+  return inside[0] < 0 ? -1 : (inside[0] ? kSolid : kFluid);
+}
+
 struct VoxArgs {
   const VTri* tris;
   const double* box;    // [6][ntri]
@@ -242,8 +261,8 @@ struct VoxArgs {
   const double* bounds;
   int nb;
   int n;
-  int te;               // tiles per block edge
-  int first;            // the launch's first tile (queue entry)
+  int te;               // tiles per block edge (KClassifyFew: runs per block)
+  int first;            // the launch's first tile (workgroup, queue entry)
   int channel;          // internal channel (else external obstacle)
   uint8_t* material;
   int* queue;           // cells the filters left open: index into material
@@ -416,35 +435,96 @@ __global__ __launch_bounds__(kVoxThreads) void KClassify(VoxArgs a) {
   for (int c = tid; c < kVoxCells; c += kVoxThreads) {
     const uint32_t s = st[c];
     if (!in_block(c)) continue;
-    int m;
-    if (s & kBitHit) {
-      m = kBoundary;
-    } else if (s & kBitOpen) {
-      m = -1;
-    } else {
-      // inside votes: decided when the certain axes settle the majority
-      int inside[2];
-      for (int q = 0; q < 2; ++q) {
-        int yes = 0, no = 0;
-        for (int ax = 0; ax < 3; ++ax) {
-          if (s & UnsureBit(q, ax)) continue;
-          if (s & OddBit(q, ax)) ++yes; else ++no;
-        }
-        inside[q] = yes >= 2 ? 1 : (no >= 2 ? 0 : -1);
-      }
-      if (!a.channel) {
-        m = inside[0] < 0 ? -1 : (inside[0] ? kSolid : kFluid);
-      } else if (inside[1] != 0) {
-        m = inside[1] < 0 ? -1 : kFluid;  // lumen
-      } else {
-        m = inside[0] < 0 ? -1 : (inside[0] ? kSolid : kFluid);
-      }
-    }
+    const int m = Decide(s, a.channel);
     if (m >= 0) {
       a.material[material_at(c)] = static_cast<uint8_t>(m);
     } else {
       const unsigned int slot = atomicAdd(a.queued, 1u);
       if (slot < a.room) a.queue[slot] = static_cast<int>(material_at(c));
+    }
+  }
+}
+
+// Few triangles and many blocks.  A wave takes kFewCells cells of a block, finds
+// the triangles (a lane each, so at most 64) that can matter to the layers they
+// are in, and goes through these with a thread per cell and the triangle in scalar
+// registers.  Few triangles are large ones: most tiles meet none or whole faces,
+// and a tile of KClassify pays about 5 ns for its barriers and its queue whatever it
+// finds.  A box of 12 triangles over 64,000 blocks, against KClassify: 4^3 cells
+// 0.20 / 0.99 ms, 8^3 1.34 / 3.02, 9^3 1.92 / 8.56, 16^3 9.4 / 20.8.
+//
+// Where all triangles lie in one block its waves go through them one after another,
+// some 3.6 us each (50 in one of 1,000 blocks: 0.18 ms, KClassify 0.04), so the
+// tiles must outweigh that: kFewTiles of them per triangle.
+constexpr int kVoxFew = 64;
+constexpr int kFewTiles = 512;
+constexpr int kFewCells = 256;
+__global__ __launch_bounds__(kVoxThreads) void KClassifyFew(VoxArgs a) {
+  const int lane = threadIdx.x & 63, n = a.n, cells = n * n * n;
+  const int64_t task =
+      (static_cast<int64_t>(a.first) + blockIdx.x) * (kVoxThreads / 64) +
+      __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  if (task / a.te >= a.nb) return;
+  const int b = static_cast<int>(task / a.te);
+  const int c0 = static_cast<int>(task % a.te) * kFewCells, c1 = c0 + min(kFewCells, cells - c0);
+  const double* ob = a.bounds + static_cast<size_t>(b) * 6;
+  double dx[3];
+  for (int d = 0; d < 3; ++d) dx[d] = (ob[3 + d] - ob[d]) / static_cast<double>(n);
+  // CellBounds (part_voxelizer.cpp:33-47), in the reference's operation order
+  auto low = [&](int d, int i) { return ob[d] + static_cast<double>(i) * dx[d]; };
+  const double rb[6] = {low(0, 0), low(1, 0), low(2, c0 / (n * n)),
+                        low(0, n - 1) + dx[0], low(1, n - 1) + dx[1], low(2, (c1 - 1) / (n * n)) + dx[2]};
+  int in = 0;
+  if (lane < a.ntri) {
+    double bx[6];
+    for (int d = 0; d < 6; ++d) bx[d] = a.box[d * a.ntri + lane];
+    in = Lists(bx, rb);
+  }
+  const uint64_t near = __ballot(in & 1), rays = __ballot(in & 14);
+  for (int c = c0 + lane; c < c1; c += 64) {
+    const int ijk[3] = {c % n, c / n % n, c / (n * n)};
+    double lo[3], hi[3], p[3];
+    for (int d = 0; d < 3; ++d) {
+      lo[d] = low(d, ijk[d]);
+      hi[d] = lo[d] + dx[d];
+      p[d] = 0.5 * (lo[d] + hi[d]);
+    }
+    uint32_t s = 0;
+    for (uint64_t todo = near; todo; todo &= todo - 1) {
+      const VTri& t = a.tris[__builtin_ctzll(todo)];
+      bool reach = true;
+      for (int d = 0; d < 3; ++d) reach = reach && (!(t.lo[d] <= t.hi[d]) || (hi[d] >= t.lo[d] && lo[d] <= t.hi[d]));
+      if (!reach || (s & kBitHit)) continue;
+      const int h = BoxHit<false>(lo, hi, t);
+      if (h != 0) s |= h == 1 ? kBitHit : kBitOpen;
+    }
+    if (!(s & (kBitHit | kBitOpen))) {
+      for (uint64_t todo = rays; todo; todo &= todo - 1) {
+        const VTri& t = a.tris[__builtin_ctzll(todo)];
+        if (t.degenerate) continue;
+        bool below[3], above[3];  // the centre, of the triangle's box
+        for (int d = 0; d < 3; ++d) {
+          const bool num = t.lo[d] <= t.hi[d];
+          below[d] = num && !(p[d] >= t.lo[d]);
+          above[d] = num && !(p[d] <= t.hi[d]);
+        }
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+          const int u = (ax + 1) % 3, w = (ax + 2) % 3;
+          if (above[ax] || below[u] || above[u] || below[w] || above[w]) continue;
+          const int h = RayHit<false>(p, ax, t);
+          if (h == 1) s ^= OddBit(t.mesh, ax);
+          if (h == kUnsure) s |= UnsureBit(t.mesh, ax);
+        }
+      }
+    }
+    const int m = Decide(s, a.channel);
+    const size_t at = static_cast<size_t>(b) * cells + c;
+    if (m >= 0) {
+      a.material[at] = static_cast<uint8_t>(m);
+    } else {
+      const unsigned int slot = atomicAdd(a.queued, 1u);
+      if (slot < a.room) a.queue[slot] = static_cast<int>(at);
     }
   }
 }
@@ -649,7 +729,9 @@ int VoxelizePart(int32_t num_blocks, int32_t n, const double* bounds, int64_t nu
   a.bounds = d_bounds;
   a.nb = num_blocks;
   a.n = n;
-  a.te = te;
+  const bool few = ntri <= kVoxFew && ntile >= kFewTiles * ntri;
+  constexpr int waves = kVoxThreads / 64;
+  a.te = few ? static_cast<int>((cells + kFewCells - 1) / kFewCells) : te;
   a.channel = channel ? 1 : 0;
   a.material = buf.Get<uint8_t>(total);
   a.room = static_cast<unsigned int>(std::min(total, kOpenRoom));
@@ -669,7 +751,10 @@ int VoxelizePart(int32_t num_blocks, int32_t n, const double* bounds, int64_t nu
   unsigned int queued = 0;
   auto classify = [&] {
     VOX_CHECK(hipMemset(a.queued, 0, sizeof(unsigned int)));
-    launch(KClassify, ntile, kVoxThreads);
+    if (few)
+      launch(KClassifyFew, (num_blocks * static_cast<int64_t>(a.te) + waves - 1) / waves, kVoxThreads);
+    else
+      launch(KClassify, ntile, kVoxThreads);
     VOX_CHECK(hipMemcpy(&queued, a.queued, sizeof(queued), hipMemcpyDeviceToHost));
   };
   classify();

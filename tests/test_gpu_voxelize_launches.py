@@ -9,12 +9,15 @@ from octlb_amd import geometry
 pytestmark = pytest.mark.gpu
 
 
-def test_more_tiles_than_one_launch_holds():
+@pytest.mark.parametrize("more", [0, 128])  # a thread per cell; a workgroup per tile
+def test_more_tiles_than_one_launch_holds(more):
     count, n = 2_100_000, 9
     assert count * 8 * 256 >= 2 ** 32
     at = np.stack(np.unravel_index(np.arange(count), (130, 130, 130)), -1).astype(np.float64)
     bounds = np.concatenate([at, at + 1.0], 1)
     soup = geometry.box_soup((0.3, 0.3, 0.3), (129.6, 129.6, 129.6))
+    if more:
+        soup = np.concatenate([soup, geometry.sphere_soup((500.0, 600.0, 700.0), 1.0, 8)])
     got, exact = geometry.voxelize_part(bounds, n, soup, geometry.PART_EXTERNAL_OBSTACLE)
     half = count // 2
     lo, lo_exact = geometry.voxelize_part(bounds[:half], n, soup, geometry.PART_EXTERNAL_OBSTACLE)
