@@ -196,6 +196,7 @@ struct octlb_dev {
   StatPart* d_stat_part = nullptr;
   double2* d_stat_sum = nullptr;
   int stat_chunks = 0;
+  int stat_longest = 0;  // chunk
   int* d_step = nullptr;   // [2]: double-buffered coarse-step counter
   int step_slot = 0;       // slot holding the current step's time
   int* inc_next = nullptr; // next-step slot, handed to the step's first kernel
@@ -1104,6 +1105,8 @@ void octlb_dev::Prepare() {
     if (sc.const_rho) {
       chunk = StatChunks(fast_stats ? tiles_of : cells, fast_stats, &chunk_begin);
       stat_chunks = static_cast<int>(chunk.size());
+      stat_longest = 0;
+      for (const int4& ch : chunk) stat_longest = std::max(stat_longest, ch.y - ch.x);
       d_stat_chunk = PAlloc<int4>(chunk.size());
       Upload(d_stat_chunk, chunk, stream);
       d_stat_chunk_begin = PAlloc<int>(chunk_begin.size());
@@ -1380,7 +1383,8 @@ void octlb_dev::Level(int l) {
     }
     par[l] ^= 1;
     if (a.want_stats == 1)
-      LaunchStatsFinalize(d_stats, d_stat_chunk, d_stat_chunk_begin, stat_chunks, nmembers, d_stat_sum, d_avg, stream);
+      LaunchStatsFinalize(d_stats, d_stat_chunk, d_stat_chunk_begin, stat_chunks, stat_longest, nmembers, d_stat_sum,
+                          d_avg, stream);
     if (a.want_stats == 2)
       LaunchStatsSequential(d_stat_val, d_stat_use, d_stat_chunk, d_stat_chunk_begin, stat_chunks, nmembers,
                             d_stat_part, d_avg, stream);

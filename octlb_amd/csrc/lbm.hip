@@ -594,6 +594,7 @@ __global__ __launch_bounds__(512) void KPadded(TileArgs<T> a) {
 constexpr int kStatChunk = 1024;   // cells per chunk of the ordered sum
 constexpr int kFastChunk = 4096;   // partials per chunk of the fast one
 constexpr int kFastThreads = 1024;
+constexpr int kFastShort = 1024;   // chunks up to this take kFastShort / 4 threads
 constexpr int kStatChunkThreads = 256;
 
 // Sum of a workgroup's (s, c) in a fixed order, in thread 0.
@@ -623,14 +624,58 @@ __device__ inline void GroupSum(double& s, double& c, double* rs, double* rc) {
 // (FP32).  Letting the last workgroup of a member sum its chunks costs a
 // device-scope fence in every workgroup: 24 us for 64 members of up to 96^3 cells,
 // where the two launches take 11 us (5.3 us, one launch, for 12 of up to 64^3).
+//
+// Members of up to kFastShort partials (40^3 cells) keep to four waves: a step of
+// 19 members of 32^3 cells takes 84.1 us, 85.3 with sixteen waves each; of one of
+// 8^3 cells 21.6 and 22.1.
 __device__ inline double StatAverage(double s, double c) {
   return c > 0.0 ? s / c : 1.0;  // CollideRhoStats::average (block_lattice.h:31)
 }
 
+// Sum of a chunk of at most kFastShort partials by the first kFastShort / 4
+// threads of a workgroup, in thread 0; the others come along for the barriers.
+__device__ inline double2 ShortSum(const double2* partial, const int4& ch, double* rs, double* rc) {
+  constexpr int kThreads = kFastShort / 4;
+  const int tid = threadIdx.x;
+  if (tid < kThreads) {
+    double s = 0.0, c = 0.0;
+    for (int i = ch.x + tid; i < ch.y; i += kThreads) {
+      s += partial[i].x;
+      c += partial[i].y;
+    }
+    rs[tid] = s;
+    rc[tid] = c;
+  }
+  __syncthreads();
+  for (int w = kThreads / 2; w > 0; w >>= 1) {
+    if (tid < w) {
+      rs[tid] += rs[tid + w];
+      rc[tid] += rc[tid + w];
+    }
+    __syncthreads();
+  }
+  return make_double2(rs[0], rc[0]);
+}
+
+// All members of at most kFastShort partials.  A member's sum is the same beside
+// longer ones, in KStatsSums.
+__global__ __launch_bounds__(kFastShort / 4) void KStatsSumsShort(const double2* partial, const int4* chunk,
+                                                                  double* avg) {
+  __shared__ double rs[kFastShort / 4], rc[kFastShort / 4];
+  const int4 ch = chunk[blockIdx.x];  // first partial, end, member
+  const double2 sum = ShortSum(partial, ch, rs, rc);
+  if (threadIdx.x == 0) avg[ch.z] = StatAverage(sum.x, sum.y);
+}
+
 __global__ __launch_bounds__(kFastThreads) void KStatsSums(const double2* partial, const int4* chunk,
                                                                 const int* chunk_begin, double2* sums, double* avg) {
-  __shared__ double rs[kFastThreads / 64], rc[kFastThreads / 64];
+  __shared__ double rs[kFastShort / 4], rc[kFastShort / 4];
   const int4 ch = chunk[blockIdx.x];  // first partial, end, member
+  if (ch.w == 0 && ch.y - ch.x <= kFastShort) {  // a whole member
+    const double2 sum = ShortSum(partial, ch, rs, rc);
+    if (threadIdx.x == 0) avg[ch.z] = StatAverage(sum.x, sum.y);
+    return;
+  }
   double s = 0.0, c = 0.0;
 #pragma unroll
   for (int k = 0; k < kFastChunk / kFastThreads; ++k) {
@@ -1907,8 +1952,13 @@ void LaunchTile(const TileArgs<T>& a, hipStream_t s) {
 
 static inline dim3 Grid(long long n, int bs) { return dim3(static_cast<unsigned>((n + bs - 1) / bs)); }
 
-void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, int members,
-                         double2* sums, double* avg, hipStream_t s) {
+void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, int longest,
+                         int members, double2* sums, double* avg, hipStream_t s) {
+  if (longest <= kFastShort) {
+    hipLaunchKernelGGL(KStatsSumsShort, dim3(nchunk), dim3(kFastShort / 4), 0, s,
+                       reinterpret_cast<const double2*>(partial), chunk, avg);
+    return;
+  }
   hipLaunchKernelGGL(KStatsSums, dim3(nchunk), dim3(kFastThreads), 0, s,
                      reinterpret_cast<const double2*>(partial), chunk, chunk_begin, sums, avg);
   if (nchunk > members)

@@ -490,9 +490,10 @@ void LaunchTile(const TileArgs<T>& a, hipStream_t s);
 // ConstRho averages of the members.  Both sums go by chunks of a member's
 // partials (fast) or cells (reference order): (first, end, member, how many of
 // the member's before it), member m owning begin[m] .. begin[m + 1] and chunks
-// [chunk_begin[m], chunk_begin[m + 1]); sums and part hold one entry per chunk.
-void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, int members,
-                         double2* sums, double* avg, hipStream_t s);
+// [chunk_begin[m], chunk_begin[m + 1]), the longest of `longest` partials; sums
+// and part hold one entry per chunk.
+void LaunchStatsFinalize(const double* partial, const int4* chunk, const int* chunk_begin, int nchunk, int longest,
+                         int members, double2* sums, double* avg, hipStream_t s);
 struct StatPair {
   long long d0, d1;  // what the chunk adds to an even / odd integer sum
 };

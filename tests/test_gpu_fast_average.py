@@ -44,3 +44,16 @@ def test_matches_the_ordered_average(sizes, precision):
                                                                        for m in range(len(sizes))]
     for s in (fast, ordered, again):
         s.close()
+
+
+@pytest.mark.parametrize("n", [8, 40])
+def test_a_member_beside_longer_ones(n):
+    """Members of up to 1,024 partials go to a smaller kernel when all are: the
+    same sum, bit for bit, as among longer ones."""
+    alone, beside = _solver((n,), 64, 1), _solver((n, 72), 64, 1)
+    for s in (alone, beside):
+        s.advance(2)
+        s.advance_graph(4)
+    assert alone.member_average_rho(0) == beside.member_average_rho(0)
+    for s in (alone, beside):
+        s.close()
